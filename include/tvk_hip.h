@@ -375,8 +375,8 @@ tvk_status tvk_binary(const tvk_binary_desc* desc);
  * Supported: F32, F16 and BF16; head_dim and head_dim_v from 1 to 512 (they
  * may differ); any element strides for q, k, v, bias (zero strides
  * broadcast) and out; batch and heads up to 65535, sequences up to 2^30.
- * float16/bfloat16 with head_dim == head_dim_v in {64, 128}, unit stride along
- * the head dimension and 16-byte aligned rows run the MFMA kernels; every
+ * float16/bfloat16 with head_dim == head_dim_v, a multiple of 8 up to 128, unit
+ * stride along the head dimension and 16-byte aligned rows run the MFMA kernels; every
  * other case runs general kernels (float32 dot products over LDS-staged
  * 64-column chunks of the head dims, the same staging of P in the dtype).
  * Other cases return TVK_ERR_UNSUPPORTED. Replaces fused_forward

@@ -1,0 +1,79 @@
+"""The MFMA attention kernels at head dims other than 64 and 128: any multiple
+of 8 up to 128, padded to tiles of 32, 64, 96 or 128 columns. Both directions
+against the float64 oracle at the attention tests' tolerance (5e-3*(|ref|+1),
+one bfloat16 step on at most 1 % of the elements), over the edges of each tile
+width, ragged lengths around the 64-key tiles, and operands whose padding
+columns hold NaN (nothing past the head dim may be read into a product)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle import oracle as orc
+from tests.gemm_cases import assert_close
+from tests.test_attention_gpu import DEV, check, check_bwd, f64, rand
+
+pytestmark = pytest.mark.gpu
+
+
+# smallest, one chunk below / at / above each tile width, largest
+@pytest.mark.parametrize("dim", [8, 24, 32, 40, 56, 72, 80, 96, 104, 120])
+@pytest.mark.parametrize("causal", [False, True])
+def test_head_dims(gpu, dim, causal):
+    dtype = torch.float16 if dim % 16 else torch.bfloat16
+    q = rand((2, 4, 130, dim), dtype, dim)
+    k, v = rand((2, 2, 130, dim), dtype, dim + 1), rand((2, 2, 130, dim), dtype, dim + 2)
+    check(q, k, v, causal=causal, what=f"D {dim}")
+    check_bwd(q, k, v, causal=causal, what=f"D {dim}")
+
+
+@pytest.mark.parametrize("dim", [32, 80, 104])
+@pytest.mark.parametrize("lens", [(1, 1), (63, 65), (64, 64), (65, 127), (3, 200)])
+def test_lengths_and_bias(gpu, dim, lens):
+    dtype = torch.float16
+    n, s = lens
+    q, k, v = rand((1, 3, n, dim), dtype, 7), rand((1, 3, s, dim), dtype, 8), rand((1, 3, s, dim), dtype, 9)
+    bias = rand((1, 3, n, s), dtype, 10)
+    if n > 2:
+        bias[0, :, 2] = float("-inf")   # a row that attends to nothing
+    check(q, k, v, bias=bias, what=f"D {dim} L {n} S {s}")
+    check_bwd(q, k, v, bias=bias, what=f"D {dim} L {n} S {s}")
+    check(q, k, v, causal=True, scale=-0.2, what=f"D {dim} L {n} S {s} causal")
+
+
+@pytest.mark.parametrize("dim", [24, 80])
+def test_columns_past_the_head_dim_are_not_used(gpu, dim):
+    # views of wider rows whose further columns are NaN, head-strided underneath
+    dtype = torch.float16
+
+    def view(heads, n, seed):
+        t = torch.full((1, n, heads, dim + 8), float("nan"), dtype=dtype)
+        t[..., :dim] = rand((1, n, heads, dim), dtype, seed)
+        return t.to(DEV)[..., :dim].transpose(1, 2)
+
+    from torchvulkan_amd import _abi
+
+    q, k, v, do = view(4, 70, 1), view(2, 70, 2), view(2, 70, 3), view(4, 70, 4)
+    out, lse = _abi.attention_fwd(q, k, v, None, True)
+    grads = _abi.attention_bwd(q, k, v, out, lse, do, None, True)
+    torch.cuda.synchronize()
+    ro, _ = orc.attention(f64(q), f64(k), f64(v), None, True)
+    assert_close(f64(out), ro, dtype, "out")
+    ref = orc.attention_bwd(f64(q), f64(k), f64(v), f64(do), None, True, None, out=f64(out), round_to=orc.F16)
+    for got, want, name in zip(grads, ref, ("dq", "dk", "dv")):
+        assert_close(f64(got), want, dtype, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim", [32, 64, 80, 128])
+def test_masks_of_the_lowest_value(gpu, dtype, dim):
+    # additive masks of the dtype's lowest finite value: masked keys get no weight beside an unmasked one, and a
+    # row masked everywhere averages over its keys (the scores vanish beside the mask)
+    low = torch.finfo(dtype).min
+    q, k, v = rand((1, 2, 40, dim), dtype, 1), rand((1, 2, 70, dim), dtype, 2), rand((1, 2, 70, dim), dtype, 3)
+    bias = torch.zeros((1, 2, 40, 70), dtype=dtype)
+    bias[..., 50:] = low
+    bias[:, :, 3, 1:] = low
+    if dtype == torch.bfloat16:
+        bias[:, :, 5] = low   # in float16 the scores do not vanish beside 65504, and the row is an ordinary one
+    check(q, k, v, bias=bias, what=f"{dtype} D {dim}")

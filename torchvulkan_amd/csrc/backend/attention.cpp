@@ -1,8 +1,8 @@
 // Scaled dot-product attention on the vulkan device: the overrideable SDPA
 // backend the reference registers (src/api/ops/attention.cpp:667-761).
 // Every case runs on the device through tvk_attention_fwd / tvk_attention_bwd:
-// the MFMA kernels for float16/bfloat16 with head dims 64/128, the library's
-// general kernels for float32, other head dims, any strides, and the score
+// the MFMA kernels for float16/bfloat16 with head dims in whole 16-byte chunks
+// up to 128, the library's general kernels for float32, other head dims, any strides, and the score
 // gradient that gives the bias gradient (summed here over the bias's
 // broadcast dimensions with the device sum).
 #include "common.h"
@@ -69,7 +69,7 @@ bool library_takes(at::ScalarType dt, int64_t dim, int64_t dim_v, int64_t batch,
 // their shapes an operand without that layout is worth one dense copy.
 at::Tensor mfma_layout(const at::Tensor& t, const Sdpa& s) {
     const bool mfma = (t.scalar_type() == at::kHalf || t.scalar_type() == at::kBFloat16) && s.dim == s.dim_v &&
-                      (s.dim == 64 || s.dim == 128);
+                      s.dim <= 128 && s.dim % 8 == 0;
     if (!mfma) return t;
     bool ok = t.stride(3) == 1 && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
     for (int i = 0; i < 3; ++i) ok = ok && (t.size(i) <= 1 || t.stride(i) % 8 == 0);
