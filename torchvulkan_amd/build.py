@@ -63,6 +63,7 @@ def _run(cmd: list[str]) -> None:
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 FILE_FLAGS = {
     "attention.hip": VGPR_FORM,
+    "attention_decode.hip": VGPR_FORM,
     "attention_part.hip": VGPR_FORM,
     "calibrate.hip": VGPR_FORM,
     "gemm_dma128.hip": VGPR_FORM,
