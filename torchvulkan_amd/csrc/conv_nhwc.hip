@@ -50,7 +50,7 @@ constexpr int V_MAXTAPS = 16;
 struct ConvRing {
     const void* act;     // gathered activation, padded NHWC (x, or dy for grad input)
     const void* wt;      // permuted weight [N][T][Cs] (forward / grad input)
-    const void* dyc;     // grad weight: dy, NCHW
+    const void* dyc;     // grad weight: dy, NCHW (MODE 1) or NHWC (MODE 2)
     const void* bias;    // forward
     void* out;           // y / dx NCHW (forward, grad input); dW (grad weight, no split)
     float* part;         // grad weight partials [split][M][N]
@@ -65,7 +65,7 @@ struct ConvRing {
     int tap_h[V_MAXTAPS], tap_w[V_MAXTAPS], tap_k[V_MAXTAPS];   // row offsets and weight tap of each k tap
     int tap_off[V_MAXTAPS], wt_off[V_MAXTAPS];   // forward / grad input: byte offsets of each k tap in act and wt
     int pix_sh, pix_sw, pix_bh, pix_bw;   // row pixel (i, j) -> source origin (i*sh + bh, j*sw + bw), border included
-    Div32 wdiv;          // grad weight: division by the output width
+    Div32 wdiv, pdiv;    // grad weight: division by the output width and plane
     // output placement (forward / grad input): pixel (i, j) -> (i*osh + orh, j*osw + orw) of [n][N][Ho][Wo]
     int Ho, Wo, osh, osw, orh, orw;
     // grad weight: output pixels per image, width; k per split; taps for the dW order
@@ -108,7 +108,8 @@ __device__ inline u32x4 frag_km(uint32_t base, int row_base, int lane) {
     const int row = row_base + lane % 16;
     return *(const TVK_LDS u32x4*)(uintptr_t)(base + row * 64 + (((lane / 16) ^ swz_km(row)) * 16));
 }
-// 16x16x32 fragment of an m-contiguous tile (k-rows of 512 bytes): transposed reads
+// 16x16x32 fragment of an m-contiguous tile (k-rows of PITCH bytes): transposed reads
+template <int PITCH = 512>
 __device__ inline u32x4 frag_mn(uint32_t base, int col_base, int lane) {
     const int g = lane / 16, s = lane % 16;
     const int col = col_base + (s % 4) * 4;
@@ -117,7 +118,7 @@ __device__ inline u32x4 frag_mn(uint32_t base, int col_base, int lane) {
 #pragma unroll
     for (int rr = 0; rr < 2; ++rr) {
         const int kr = g * 8 + rr * 4 + s / 4;
-        TVK_LDS s16x4* ptr = (TVK_LDS s16x4*)(uintptr_t)(base + kr * 512 + ((chunk ^ swz_mn(kr)) * 16) + within);
+        TVK_LDS s16x4* ptr = (TVK_LDS s16x4*)(uintptr_t)(base + kr * PITCH + ((chunk ^ swz_mn(kr)) * 16) + within);
         const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ptr));
         out[rr * 2] = w.x;
         out[rr * 2 + 1] = w.y;
@@ -129,7 +130,11 @@ __device__ inline u32x4 frag_mn(uint32_t base, int col_base, int lane) {
 constexpr int ring_waves(int bm, int bn) { return bm == 256 ? (bn == 64 ? 4 : 8) : 2 * (bn / 64); }
 
 // MODE 0: rows are pixels (forward, grad input; grid z = sub-pixel phase);
-// MODE 1: grad weight (grid z = k split).
+// MODE 1: grad weight (grid z = k split), dy read from NCHW: planes of whole
+// 32-pixel stages. MODE 2: grad weight on any plane, dy channels-last, so that
+// a stage's 32 output pixels are 32 consecutive k rows whatever images they
+// belong to (both operands are m/n-contiguous tiles read back transposed);
+// rows past the last pixel read zeros.
 template <int DT, int MODE, int BM, int BN>
 __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(ConvRingSet set) {
     static_assert(MODE == 0 || BM == 256, "grad weight uses 256-row tiles");
@@ -153,19 +158,19 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
     const int m0 = blockIdx.x * V_BM, n0 = blockIdx.y * BN;
     if (m0 >= p.M) return;   // this phase has fewer row tiles than the grid
     const int z = blockIdx.z;
-    const int kb = MODE == 1 ? z * p.k_chunk : 0;
-    const int klen = MODE == 1 ? min(p.k_chunk, p.K - kb) : p.K;
-    const int nk = klen / V_BK;
+    const int kb = MODE >= 1 ? z * p.k_chunk : 0;
+    const int klen = MODE >= 1 ? min(p.k_chunk, p.K - kb) : p.K;
+    const int nk = (klen + V_BK - 1) / V_BK;
 
     const i32x4 ra = v_rsrc(p.act, p.act_bytes);
-    const i32x4 rb = v_rsrc(MODE == 1 ? p.dyc : p.wt, MODE == 1 ? p.dyc_bytes : p.wt_bytes);
+    const i32x4 rb = v_rsrc(MODE >= 1 ? p.dyc : p.wt, MODE >= 1 ? p.dyc_bytes : p.wt_bytes);
 
     // ---- per-lane, per-load constants ----
     // Rows past M (pixels, or (tap, channel) rows) and columns past N read a
     // valid row instead; their results are never stored.
     // A (MODE 0): KM tile, 16 rows per block; a_off = byte offset of the row
     //   pixel's origin and the lane's 8 channels, a stage adds its tap and channel
-    // A (MODE 1): MN tile, 2 k-rows per block; a_off = element offset of the
+    // A (MODE 1, 2): MN tile, 2 k-rows per block; a_off = element offset of the
     //   lane's (tap, channel) chunk, a stage adds its output pixel's position
     int a_off[DA], a_kr[DA];
 #pragma unroll
@@ -189,10 +194,17 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
         }
     }
     // B: KM tile, 16 rows (output channels) per block; byte offset of the lane's row and chunk
+    // (MODE 2: MN tile, k rows of BN channels; columns past N read zeros)
     int b_off[DB];
 #pragma unroll
     for (int q = 0; q < DB; ++q) {
         const int blk = wave * DB + q;
+        if constexpr (MODE == 2) {
+            const int kr = blk * (512 / BN) + lane / (BN / 8);
+            const int n = n0 + ((lane % (BN / 8)) ^ swz_mn(kr)) * 8;
+            b_off[q] = n < p.N ? ((kb + kr) * p.N + n) * 2 : (int)kOOB;
+            continue;
+        }
         const int row = blk * 16 + lane / 4;
         const int n = min(n0 + row, p.N - 1);
         const int bc = ((lane % 4) ^ swz_km(row)) * 8;
@@ -216,6 +228,20 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
                 ic0 = 0;
                 ++it;
             }
+        } else if constexpr (MODE == 2) {
+            const int k0 = kb + s * V_BK;
+#pragma unroll
+            for (int q = 0; q < DA; ++q) {
+                const int k = k0 + a_kr[q];
+                const int img = (int)div32((uint32_t)k, p.pdiv), o = k - img * p.HWo;
+                const int oh = (int)div32((uint32_t)o, p.wdiv), ow = o - oh * p.Wd;
+                const int off = ((img * p.Hs + oh * p.pix_sh) * p.Ws + ow * p.pix_sw) * p.Cs + a_off[q];
+                v_dma16(ra, slot + (uint32_t)((wave * DA + q) * 1024), k < p.K ? (uint32_t)off * 2 : kOOB);
+            }
+            // dy rows past the last pixel lie past the buffer
+#pragma unroll
+            for (int q = 0; q < DB; ++q)
+                v_dma16(rb, slot + OPA + (uint32_t)((wave * DB + q) * 1024), (uint32_t)b_off[q] + (uint32_t)(s * V_BK * p.N * 2));
         } else {
             // the stage's 32 output pixels lie in one image (HWo % 32 == 0)
             const int k0 = kb + s * V_BK;
@@ -244,6 +270,10 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
         if constexpr (MODE == 0) return frag_km(st, wm * WTM + i * 16, lane);
         else return frag_mn(st, wm * WTM + i * 16, lane);
     };
+    auto read_b = [&](uint32_t st, int j) {
+        if constexpr (MODE == 2) return frag_mn<BN * 2>(st + OPA, wn * 64 + j * 16, lane);
+        else return frag_km(st + OPA, wn * 64 + j * 16, lane);
+    };
     u32x4 fa[2][FM], fb[2][FN];
     if (nk > 0) {
 #pragma unroll
@@ -254,7 +284,7 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
 #pragma unroll
         for (int i = 0; i < FM; ++i) fa[0][i] = read_a(lds0, i);
 #pragma unroll
-        for (int j = 0; j < FN; ++j) fb[0][j] = frag_km(lds0 + OPA, wn * 64 + j * 16, lane);
+        for (int j = 0; j < FN; ++j) fb[0][j] = read_b(lds0, j);
         if (nk >= V_NS) v_wait<DS * (V_NS - 2)>(); else v_wait<0>();
         __syncthreads();
 
@@ -269,7 +299,7 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
                 if (q % 2 == 0) {
                     const int r = q / 2;
                     if (r < FM) fa[cur ^ 1][r] = read_a(st_next, r);
-                    else if (r < FM + FN) fb[cur ^ 1][r - FM] = frag_km(st_next + OPA, wn * 64 + (r - FM) * 16, lane);
+                    else if (r < FM + FN) fb[cur ^ 1][r - FM] = read_b(st_next, r - FM);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -289,7 +319,7 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
     }
 
     typedef typename elem<DT>::T T;
-    if constexpr (MODE == 1) {
+    if constexpr (MODE >= 1) {
         // (tap, channel) rows x output-channel columns: partials, or dW[co][c][t]
 #pragma unroll
         for (int i = 0; i < FM; ++i)
@@ -377,12 +407,17 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
 // input). Column block nx - 1, when the plane has a border, zeroes the border
 // pixels of its channels (the rows above and below, then the columns left and
 // right of each image row); the others copy 64 channels x PX pixels.
-// VEC (HW % 8 == 0, C % 8 == 0): PX = 256, no LDS. A lane loads 8 pixels of 8
-// channels (eight 16-byte loads; 8 lanes read 128 contiguous bytes of a channel
-// row), transposes the 8x8 block of 16-bit elements in registers and stores 8
-// pixels of 8 channels (8 lanes write 128 contiguous bytes of a pixel).
-// Otherwise PX = 64 through an LDS tile, element accesses where the counts
-// leave no 16-byte run.
+// VEC (C % 8 == 0): PX = 256, no LDS. A lane loads 8 pixels of 8 channels
+// (eight 16-byte loads; 8 lanes read 128 contiguous bytes of a channel row),
+// transposes the 8x8 block of 16-bit elements in registers and stores 8 pixels
+// of 8 channels (8 lanes write 128 contiguous bytes of a pixel). The loads
+// need no alignment beyond the element's, so any plane takes this path (14 x
+// 14 and 7 x 7 planes went through LDS one element at a time: 12-15 us for
+// 32 x 256 x 14 x 14 and its weight, 8-9 here); the last chunk of a plane whose
+// pixels are no multiple of 8 goes element by element.
+// Otherwise PX = 64 through an LDS tile, element accesses.
+// A grad weight's launch copies two tensors: workgroups past the first
+// tensor's take the second's.
 struct WeightPermute {
     const uint16_t* w = nullptr;
     uint16_t* out = nullptr;
@@ -394,6 +429,10 @@ struct NhwcArgs {
     uint16_t* dst;
     int C, H, W, Hs, Ws, pt, pl;
     int nblk, nx, cy, copy_blocks;   // copy column blocks per plane (nblk, plus 1 with a border)
+};
+
+struct NhwcSet {
+    NhwcArgs t[2];       // copy_blocks 0: none
     WeightPermute wp;
 };
 
@@ -431,13 +470,23 @@ __device__ inline void zero_border(const NhwcArgs& a, uint16_t* d, int c0, bool 
     }
 }
 
+// 16 bytes from an address with the element's alignment only
+__device__ inline u32x4 load16_any(const uint16_t* p) {
+    u32x4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+
 template <bool VEC>
-__global__ __launch_bounds__(256) void nchw_to_nhwc_kernel(NhwcArgs a) {
-    const int b = blockIdx.x;
-    if (b >= a.copy_blocks) {
-        permute_weight(a.wp, b - a.copy_blocks, (int)gridDim.x - a.copy_blocks);
+__global__ __launch_bounds__(256) void nchw_to_nhwc_kernel(NhwcSet set) {
+    int b = blockIdx.x;
+    const int copies = set.t[0].copy_blocks + set.t[1].copy_blocks;
+    if (b >= copies) {
+        permute_weight(set.wp, b - copies, (int)gridDim.x - copies);
         return;
     }
+    const NhwcArgs& a = set.t[b < set.t[0].copy_blocks ? 0 : 1];
+    if (b >= set.t[0].copy_blocks) b -= set.t[0].copy_blocks;
     const int bx = b % a.nx, img = b / (a.nx * a.cy), c0 = (b / a.nx - img * a.cy) * 64;
     const int C = a.C, W = a.W, HW = a.H * a.W;
     uint16_t* d = a.dst + (int64_t)img * a.Hs * a.Ws * C;
@@ -452,11 +501,23 @@ __global__ __launch_bounds__(256) void nchw_to_nhwc_kernel(NhwcArgs a) {
         const int px = bx * 256 + wave * 64 + (lane / 8) * 8;
         if (c >= C || px >= HW) return;
         u32x4 r[8];
+        if (px + 8 <= HW) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) r[i] = *reinterpret_cast<const u32x4*>(s + (int64_t)(c + i) * HW + px);
+            for (int i = 0; i < 8; ++i) r[i] = load16_any(s + (int64_t)(c + i) * HW + px);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint16_t* q = s + (int64_t)(c + i) * HW + px + 2 * e;
+                    const uint32_t lo = px + 2 * e < HW ? q[0] : 0, hi = px + 2 * e + 1 < HW ? q[1] : 0;
+                    r[i][e] = lo | (hi << 16);
+                }
+        }
         int h = px / W, w = px - h * W;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
+            if (px + j >= HW) break;
             // pixel px + j: channel pairs (2k, 2k + 1) packed low/high
             uint32_t v[4];
 #pragma unroll
@@ -535,8 +596,8 @@ __global__ __launch_bounds__(256) void wgrad_ring_reduce_kernel(const float* par
     }
 }
 
-// Launches MODE 0 over set.ph[0..nph) (grid z = phase) or MODE 1 over `splits`
-// k splits. 128-row tiles when 256-row tiles would leave the device under-filled.
+// Launches MODE 0 over set.ph[0..nph) (grid z = phase) or MODE 1 or 2 over
+// `splits` k splits. 128-row tiles when 256-row tiles would leave the device under-filled.
 #ifndef TVK_RING_MIN_BN
 #define TVK_RING_MIN_BN 64
 #endif
@@ -569,29 +630,42 @@ struct Border {
     int pt = 0, pb = 0, pl = 0, pr = 0;
 };
 
-void launch_nhwc(const void* src, void* dst, int n, int C, int H, int W, const Border& bd, hipStream_t s,
-                 const WeightPermute& wp = WeightPermute()) {
-    NhwcArgs a;
-    a.src = static_cast<const uint16_t*>(src);
-    a.dst = static_cast<uint16_t*>(dst);
-    a.C = C; a.H = H; a.W = W;
-    a.Hs = H + bd.pt + bd.pb; a.Ws = W + bd.pl + bd.pr;
-    a.pt = bd.pt; a.pl = bd.pl;
-    // 16-byte accesses: every channel row and pixel starts 16-byte aligned (the
-    // source is, and the workspace is 256-byte aligned)
-    const bool vec = (H * W) % 8 == 0 && C % 8 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
+// One tensor of a layout copy: [n][C][H][W] at src to bordered NHWC at dst.
+struct NhwcCopy {
+    const void* src;
+    void* dst;
+    int C, H, W;
+    Border bd;
+};
+
+void launch_nhwc(const NhwcCopy* copies, int count, int n, hipStream_t s, const WeightPermute& wp = WeightPermute()) {
+    NhwcSet set;
+    memset(&set.t, 0, sizeof(set.t));
+    bool vec = true;
+    for (int i = 0; i < count; ++i) vec = vec && copies[i].C % 8 == 0;
     const int px = vec ? 256 : 64;
-    a.nblk = (H * W + px - 1) / px;
-    const bool border = a.Hs > H || a.Ws > W;
-    a.nx = a.nblk + (border ? 1 : 0);
-    a.cy = (C + 63) / 64;
-    a.copy_blocks = a.nx * a.cy * n;
-    a.wp = wp;
+    int blocks = 0;
+    for (int i = 0; i < count; ++i) {
+        const NhwcCopy& q = copies[i];
+        NhwcArgs& a = set.t[i];
+        a.src = static_cast<const uint16_t*>(q.src);
+        a.dst = static_cast<uint16_t*>(q.dst);
+        a.C = q.C; a.H = q.H; a.W = q.W;
+        a.Hs = q.H + q.bd.pt + q.bd.pb; a.Ws = q.W + q.bd.pl + q.bd.pr;
+        a.pt = q.bd.pt; a.pl = q.bd.pl;
+        a.nblk = (q.H * q.W + px - 1) / px;
+        const bool border = a.Hs > q.H || a.Ws > q.W;
+        a.nx = a.nblk + (border ? 1 : 0);
+        a.cy = (q.C + 63) / 64;
+        a.copy_blocks = a.nx * a.cy * n;
+        blocks += a.copy_blocks;
+    }
+    set.wp = wp;
     const int64_t wn = (int64_t)wp.cout * wp.cin * wp.taps;
     const int wblocks = wp.w ? (int)std::min<int64_t>((wn + 255) / 256, 1024) : 0;
-    const dim3 grid((unsigned)(a.copy_blocks + wblocks));
-    if (vec) hipLaunchKernelGGL(nchw_to_nhwc_kernel<true>, grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(nchw_to_nhwc_kernel<false>, grid, dim3(256), 0, s, a);
+    const dim3 grid((unsigned)(blocks + wblocks));
+    if (vec) hipLaunchKernelGGL(nchw_to_nhwc_kernel<true>, grid, dim3(256), 0, s, set);
+    else hipLaunchKernelGGL(nchw_to_nhwc_kernel<false>, grid, dim3(256), 0, s, set);
 }
 
 // Border that keeps rows lo + i*step + [tap_lo, tap_hi] for i in [0, count)
@@ -2027,7 +2101,8 @@ bool conv_ring_applies(const tvk_conv_desc& d, int mode) {
     auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
     if (!al16(d.x) || !al16(d.weight) || !al16(d.y)) return false;
     if (mode == 1 && (d.stride[0] > 4 || d.stride[1] > 4)) return false;
-    if (mode == 2 && (d.h_out * d.w_out) % 32 != 0) return false;
+    // planes of other than whole 32-pixel stages read dy channels-last, in 8-channel chunks
+    if (mode == 2 && (d.h_out * d.w_out) % 32 != 0 && d.c_out % 8 != 0) return false;
     // 32-bit element offsets inside the kernels
     const int64_t big = std::max({d.n * d.c_in * d.h * d.w, d.n * d.c_out * d.h_out * d.w_out, d.c_out * d.c_in * d.kh * d.kw});
     return big < (int64_t(1) << 30);
@@ -2090,7 +2165,8 @@ tvk_status conv_ring_run(const tvk_conv_desc& d, int mode, const char* who) {
         wp.w = static_cast<const uint16_t*>(d.weight);
         wp.out = reinterpret_cast<uint16_t*>(ws + act_b);
         wp.cout = cout; wp.cin = cin; wp.taps = T; wp.forward = mode == 0;
-        launch_nhwc(src, ws, n, Cs, H0, W0, bd, s, wp);
+        const NhwcCopy act{src, ws, Cs, H0, W0, bd};
+        launch_nhwc(&act, 1, n, s, wp);
         p.act = ws;
         p.wt = ws + act_b;
         p.Hs = Hs; p.Ws = Ws; p.Cs = Cs;
@@ -2165,14 +2241,18 @@ tvk_status conv_ring_run(const tvk_conv_desc& d, int mode, const char* who) {
             flush();
         }
     } else {
-        // grad weight: x to bordered NHWC; dy read NCHW; K = output pixels split into partials
+        // grad weight: x to bordered NHWC; dy read NCHW where a stage's 32 pixels lie in one image, else copied
+        // channels-last with x in one launch (the element-gathering kernel of conv.hip took such planes before:
+        // bfloat16 32 x 128 x 28 x 28 to 128 channels, 3x3: 132 us there; 36 here, 22 of them the products); K =
+        // output pixels split into partials
+        const bool dy_last = (Ho * Wo) % 32 != 0;
         Border bd;
         border_for(-ph, sh, Ho, 0, (kh - 1) * dh, H, bd.pt, bd.pb);
         border_for(-pw, sw, Wo, 0, (kw - 1) * dw, W, bd.pl, bd.pr);
         const int Hs = H + bd.pt + bd.pb, Ws = W + bd.pl + bd.pr;
         if ((size_t)n * cin * Hs * Ws * es >= ((size_t)1 << 31))
             return fail(TVK_ERR_UNSUPPORTED, std::string(who) + ": the bordered channels-last copy exceeds 2 GiB");
-        const size_t act_b = align((size_t)n * cin * Hs * Ws * es);
+        const size_t act_b = align((size_t)n * cin * Hs * Ws * es), dy_b = dy_last ? align((size_t)n * cout * Ho * Wo * es) : 0;
         p.M = T * cin;
         p.N = cout;
         p.K = n * Ho * Wo;
@@ -2189,12 +2269,13 @@ tvk_status conv_ring_run(const tvk_conv_desc& d, int mode, const char* who) {
         int64_t chunk = ((p.K + split - 1) / split + V_BK - 1) / V_BK * V_BK;
         split = (p.K + chunk - 1) / chunk;
         const size_t part_b = split > 1 ? (size_t)split * p.M * p.N * 4 : 0;
-        char* ws = static_cast<char*>(scratch.get(act_b + part_b, s));
+        char* ws = static_cast<char*>(scratch.get(act_b + dy_b + part_b, s));
         if (!ws) return fail(TVK_ERR_OOM, std::string(who) + ": no workspace for the channels-last copy");
-        launch_nhwc(d.x, ws, n, cin, H, W, bd, s);
+        const NhwcCopy copies[2] = {{d.x, ws, cin, H, W, bd}, {d.y, ws + act_b, cout, Ho, Wo, Border()}};
+        launch_nhwc(copies, dy_last ? 2 : 1, n, s);
         p.act = ws;
-        p.dyc = d.y;
-        p.part = split > 1 ? reinterpret_cast<float*>(ws + act_b) : nullptr;
+        p.dyc = dy_last ? ws + act_b : d.y;
+        p.part = split > 1 ? reinterpret_cast<float*>(ws + act_b + dy_b) : nullptr;
         p.out = d.weight;
         p.Hs = Hs; p.Ws = Ws; p.Cs = cin;
         p.ntap = T;
@@ -2203,13 +2284,19 @@ tvk_status conv_ring_run(const tvk_conv_desc& d, int mode, const char* who) {
         p.pix_sh = sh; p.pix_sw = sw;
         p.HWo = Ho * Wo; p.Wd = Wo; p.kh_kw = T;
         p.wdiv = make_div((uint32_t)Wo);
+        p.pdiv = make_div((uint32_t)(Ho * Wo));
         p.k_chunk = (int)chunk; p.split = (int)split;
         p.act_bytes = (int)((size_t)n * cin * Hs * Ws * es);
         p.dyc_bytes = (int)((size_t)n * cout * Ho * Wo * es);
         ConvRingSet set;
         set.ph[0] = p;
-        if (f16) launch_ring<TVK_F16, 1>(set, 1, (int)split, s);
-        else launch_ring<TVK_BF16, 1>(set, 1, (int)split, s);
+        if (dy_last) {
+            if (f16) launch_ring<TVK_F16, 2>(set, 1, (int)split, s);
+            else launch_ring<TVK_BF16, 2>(set, 1, (int)split, s);
+        } else {
+            if (f16) launch_ring<TVK_F16, 1>(set, 1, (int)split, s);
+            else launch_ring<TVK_BF16, 1>(set, 1, (int)split, s);
+        }
         if (split > 1) {
             // group count: enough workgroups to fill the device, at most the splits
             const int total = p.M * p.N;
