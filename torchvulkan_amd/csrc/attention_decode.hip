@@ -433,21 +433,17 @@ void attn_decode_fwd(int dtype, const AttnArgs& args, bool bias, int64_t batch, 
     p.splits = (tiles + p.per - 1) / p.per;
     Scratch scratch;
     if (p.splits > 1) {
-        // Partials need scratch. A captured launch may be replayed on another stream, where the pool's ownership by
-        // stream does not hold, and must not allocate: it takes one split, as do a call that gets no memory and one on
-        // hipStreamPerThread, a handle that stands for a stream of each thread.
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        const bool capturing = s == hipStreamPerThread || hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
-        if (capturing) (void)hipGetLastError();
+        // partials need scratch: a call that gets none takes one split
+        const bool can = scratch_usable(s);
         const size_t rows = (size_t)p.splits * all_rows, bytes = rows * (args.hd + 2) * 4;
-        float* part = capturing || bytes >= (size_t)1 << 31 ? nullptr : static_cast<float*>(scratch.get(bytes, s));
+        float* part = !can || bytes >= (size_t)1 << 31 ? nullptr : static_cast<float*>(scratch.get(bytes, s));
         if (part) {
             p.part_o = part;
             p.part_ml = part + rows * args.hd;
             p.part_bytes = (unsigned)bytes;
             p.count = split_counters(s, base);
         } else {
-            if (!capturing) clear_error();
+            clear_error();
             p.splits = 1;
             p.per = tiles;
         }

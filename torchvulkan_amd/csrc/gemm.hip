@@ -772,7 +772,7 @@ Plan with_kern(Plan pl, Kern k, const char* name) {
     return pl;
 }
 
-// The M <= 16 streaming kernel on a laid-out plan (no repacks: the layout
+// The streaming kernels of few rows (gemm_skinny.hip) on a laid-out plan (no repacks: the layout
 // never repacks such a product); it loads A by rows of k, so 16-byte loads
 // need A k-contiguous too.
 Plan skinny_plan(const tvk_gemm_desc& d, Plan pl) {
@@ -818,6 +818,8 @@ Plan make_plan(const tvk_gemm_desc& d) {
     if (d.K == 0) return Plan{Kern::K0, true, true, true, "gemm_k0_fill"};
     if (!plan_layout(d, pl)) return pl;
     if (d.dtype != TVK_F32 && !(d.flags & TVK_GEMM_EXACT) && skinny_applies(d.M, d.N, d.K, d.batch))
+        return skinny_plan(d, pl);
+    if (d.dtype != TVK_F32 && !(d.flags & TVK_GEMM_EXACT) && skinny_wide_applies(make_args(d), pl.bk, pl.vec && pl.ak))
         return skinny_plan(d, pl);
     const int64_t t256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * d.batch;
     const bool big = d.M >= 256 && d.N >= 256 && t256 >= 192;
@@ -932,7 +934,8 @@ std::vector<Plan> candidate_plans(const tvk_gemm_desc& d) {
         add(with_kern(lay, Kern::SEQ16, "gemm_seq_mfma_64x64"));
         return out;
     }
-    if (skinny_applies(d.M, d.N, d.K, d.batch)) add(skinny_plan(d, lay));
+    if (skinny_applies(d.M, d.N, d.K, d.batch) || skinny_wide_applies(make_args(d), lay.bk, lay.vec && lay.ak))
+        add(skinny_plan(d, lay));
     add(with_kern(lay, Kern::MFMA128, "gemm16_mfma_128x128"));
     add(with_kern(lay, Kern::MFMA64, "gemm16_mfma_64x64"));
     for (int64_t want : {2, 4, 8, 16}) {
@@ -1090,7 +1093,8 @@ tvk_status run(const tvk_gemm_desc& d, const Plan& pl, hipStream_t s, char* fixe
         const int64_t a_rows = pl.ak ? d.M : d.K, a_ld = repack_ld(pl.ak ? d.K : d.M, pl.ak);
         const int64_t b_rows = pl.bk ? d.N : d.K, b_ld = repack_ld(pl.bk ? d.K : d.N, pl.bk);
         size_t rep_a = 0, rep_b = 0;
-        const size_t need = plan_scratch_bytes(d, pl, nb, &rep_a, &rep_b);
+        size_t need = plan_scratch_bytes(d, pl, nb, &rep_a, &rep_b);
+        if (pl.kern == Kern::SKINNY && !fixed) need = 0;   // launch_skinny leases its own
         char* ws = nullptr;
         Scratch scratch;
         if (fixed) {

@@ -464,5 +464,7 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
 size_t skinny_scratch_bytes(const GemmArgs& p, bool b_kmajor, bool vec);
 const char* skinny_name(const GemmArgs& p, bool b_kmajor, bool vec);
 bool skinny_applies(int64_t M, int64_t N, int64_t K, int64_t batch);
+// The k-contiguous form's products above skinny_applies' 16 rows: up to 64 rows, no repacks.
+bool skinny_wide_applies(const GemmArgs& p, bool b_kmajor, bool vec);
 
 }  // namespace tvk

@@ -10,7 +10,8 @@
 // columns against the 16 rows of A. B stored k-contiguous ([N][K], a transposed
 // weight view) is loaded straight into MFMA operands; B stored n-contiguous
 // ([K][N]) is written to a wave-private LDS tile as it arrives and read back
-// along k.
+// along k. It runs the layouts without 16-byte rows, and n-contiguous B where
+// the ring below does not apply.
 //
 // B n-contiguous with 16-byte aligned rows ([K][N], the C5 layout) takes a
 // second kernel, gemm16_skinny_ring: workgroups of 8 waves own 128 columns
@@ -288,6 +289,185 @@ int ring_splits(const GemmArgs& p) {
     return split;
 }
 
+// ---------------------------------------------------------------------------
+// The ring for B k-contiguous (nn.Linear's weight [N][K]) with 16-byte rows, M <= 64
+// ---------------------------------------------------------------------------
+// Bound by reading B once, as the ring above; what the split has to get right
+// is how B's rows meet the memory channels.
+//   - A workgroup of 8 waves owns 64 columns: four 16-column groups x two k
+//     halves of a 256-k stage, so a stage reads 512 bytes of each of 64 rows
+//     (the direct-to-register kernel read 64-byte pieces: 3.9 TB/s on bfloat16
+//     16 x 4096 x 14336, 30.6 us). B and A arrive by buffer loads straight into
+//     a ring of 2-4 stages; each wave reads only its own 4 KB of a B stage, A
+//     is shared. The halves' sums meet in LDS at the end. 128 columns and one
+//     k half (256 bytes a row, and twice as many K chunks for the same
+//     workgroups) took 27.4 us where this takes 22.8 (5.2 TB/s).
+//   - With rows a multiple of 4 KB apart the same stage of every row lies on
+//     the same channels, of memory and of an XCD's L2: workgroups start their
+//     k loop at different stages, counted so that the workgroups of one XCD
+//     (every eighth) take all of them (26.8 -> 22.8 us there; 8192 x 8192
+//     44 us with the workgroups of an XCD on two stages, 35.6 unrotated, 26.7
+//     so). A fixed order for a shape: the same bits every run.
+//   - K is split between workgroups up to about one per CU in chunks of at
+//     least four stages (the exchange costs about 1.5 us: 7 x 1000 -> 500 takes
+//     5.2 us whole, 6.2 in two), summed by the last workgroup of a strip
+//     (split_fixup) or a second launch.
+//   - MF 16-row blocks of A: up to 64 rows (4096 -> 14336: 24.3 us for 32 rows,
+//     31.7 for 64; the split 128 x 128 ring took 33.1 and 36.8). Above 32 rows A
+//     weighs as much as B in the ring, and from K = 8192 the 128 x 128 tiles
+//     are as fast (64 x 14336 x 4096: 32.7 us there, 34.2 here).
+constexpr int SKR_K = 128;                   // k per wave and stage: 256 bytes of each row
+constexpr int SKR_KG = 2;                    // k groups of a workgroup
+constexpr int SKR_NB = 16 * SR_NW / SKR_KG;  // columns of a workgroup
+constexpr int SKR_KST = SKR_K * SKR_KG;      // k per stage
+constexpr int SKR_B = SR_NW * 16 * SKR_K * 2;   // B bytes per stage: 32 KB, 4 KB per wave
+
+// LDS bytes of a stage (MF 16-row blocks of A) and ring depth in 160 KB
+constexpr int kring_stage(int mf) { return SKR_B + mf * SKR_KG * 4096; }
+constexpr int kring_depth(int mf) { return std::min(4, 160 * 1024 / kring_stage(mf)); }
+
+template <int DT, int MF>
+__global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs p) {
+    constexpr int CG = SR_NW / SKR_KG;   // 16-column groups
+    constexpr int NS = kring_depth(MF), STB = kring_stage(MF);
+    constexpr int AL = 4 * MF * SKR_KG / SR_NW;   // A loads per wave
+    static_assert(AL * SR_NW == 4 * MF * SKR_KG, "whole loads");
+    __shared__ __attribute__((aligned(1024))) char lds_raw[NS * STB];
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TVK_LDS char*)lds_raw);
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int cg = wave % CG, kg = wave / CG;
+    const int n0 = blockIdx.x * SKR_NB, z = blockIdx.y, b = blockIdx.z;
+    const int kb = p.split > 1 ? z * p.k_chunk : 0;
+    const int kend = p.split > 1 ? min(p.K, kb + p.k_chunk) : p.K;
+    const int nk = (kend - kb + SKR_KST - 1) / SKR_KST;
+    const int rot = p.sb[2] % 2048 == 0 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)nk) : 0;
+
+    const char* A = reinterpret_cast<const char*>(p.a) + a_boff(p, b) * 2;
+    const char* B = reinterpret_cast<const char*>(p.b) + b_boff(p, b) * 2;
+    const i32x4 ra = sr_rsrc(A, 2 * ((int64_t)(p.M - 1) * p.sa[1] + p.K));
+    const i32x4 rb = sr_rsrc(B, 2 * ((int64_t)(p.N - 1) * p.sb[2] + p.K));
+    // a load brings 4 rows of 256 bytes; LDS slot c of row r holds 16-byte chunk c ^ (r % 16)
+    uint32_t b_off[4], a_off[AL];
+    int b_k[4], a_k[AL];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const int row = 4 * q + lane / 16, n = n0 + cg * 16 + row;
+        b_k[q] = kg * SKR_K + ((lane % 16) ^ row) * 8;
+        b_off[q] = n < p.N ? (uint32_t)(((int64_t)n * p.sb[2] + kb + b_k[q]) * 2) : kOOB;
+    }
+#pragma unroll
+    for (int q = 0; q < AL; ++q) {
+        const int blk = wave * AL + q, row = (blk % (4 * MF)) * 4 + lane / 16;
+        a_k[q] = blk / (4 * MF) * SKR_K + ((lane % 16) ^ (row % 16)) * 8;
+        a_off[q] = row < p.M ? (uint32_t)(((int64_t)row * p.sa[1] + kb + a_k[q]) * 2) : kOOB;
+    }
+    auto issue = [&](int s) {
+        if (s >= nk) return;
+        const uint32_t slot = lds0 + (uint32_t)((s % NS) * STB);
+        int ks = s + rot;
+        if (ks >= nk) ks -= nk;
+        const int left = p.K - kb - ks * SKR_KST;   // chunks at or past it would read the next row: zeros instead
+        const uint32_t step = (uint32_t)(ks * SKR_KST * 2);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            sr_dma16(rb, slot + (uint32_t)(wave * 4096 + q * 1024), b_k[q] < left ? b_off[q] + step : kOOB);
+#pragma unroll
+        for (int q = 0; q < AL; ++q)
+            sr_dma16(ra, slot + SKR_B + (uint32_t)((wave * AL + q) * 1024), a_k[q] < left ? a_off[q] + step : kOOB);
+    };
+
+    f32x4 acc[MF];
+#pragma unroll
+    for (int m = 0; m < MF; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < NS - 1; ++s) issue(s);
+    const int g = lane / 16, c16 = lane % 16;
+    for (int kt = 0; kt < nk; ++kt) {
+        // stage kt landed; the stages issued after it may be in flight
+        if (nk - 1 - kt >= NS - 2) sr_wait<(4 + AL) * (NS - 2)>();
+        else sr_wait<0>();
+        __syncthreads();
+        issue(kt + NS - 1);
+        const uint32_t st = lds0 + (uint32_t)((kt % NS) * STB);
+#pragma unroll
+        for (int ks = 0; ks < SKR_K / 32; ++ks) {
+            const uint32_t at = (uint32_t)(c16 * 256 + (((ks * 4 + g) ^ c16) * 16));
+            const u32x4 bf = *(const TVK_LDS u32x4*)(uintptr_t)(st + wave * 4096 + at);
+#pragma unroll
+            for (int m = 0; m < MF; ++m) {
+                const u32x4 af = *(const TVK_LDS u32x4*)(uintptr_t)(st + SKR_B + (kg * MF + m) * 4096 + at);
+                acc[m] = mfma16<DT>(af, bf, acc[m]);
+            }
+        }
+    }
+    sr_wait<0>();
+    // the second k half's sums onto the first's
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(lds_raw);
+    if (kg > 0) {
+#pragma unroll
+        for (int m = 0; m < MF; ++m) red[(cg * MF + m) * 64 + lane] = acc[m];
+    }
+    __syncthreads();
+    if (kg == 0) {
+#pragma unroll
+        for (int m = 0; m < MF; ++m) acc[m] += red[(cg * MF + m) * 64 + lane];
+    }
+
+    // lane l holds column l % 16 of the wave's 16, rows 16 m + (l / 16) * 4 + r
+    const int n = n0 + cg * 16 + c16;
+    if (kg == 0 && n < p.N) {
+#pragma unroll
+        for (int m = 0; m < MF; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = m * 16 + g * 4 + r;
+                if (row >= p.M) continue;
+                const int64_t pi = (((int64_t)z * p.batch + b) * p.M + row) * p.N + n;
+                if (p.split > 1 && p.tile_count) part_store(part_rsrc(p), pi, acc[m][r]);
+                else if (p.split > 1) p.part[pi] = acc[m][r];
+                else store_out<DT, true>(p, b, row, n, acc[m][r]);
+            }
+    }
+    if (p.split > 1 && p.tile_count)
+        split_fixup<DT, 64 * SR_NW, 16 * MF, SKR_NB>(p, b, 0, n0, p.tile_count + (int64_t)b * gridDim.x + blockIdx.x,
+                                                   reinterpret_cast<int*>(lds_raw));
+}
+
+bool kring_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
+    auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
+    if (!b_kmajor || !vec || !al16(p.a) || !al16(p.b) || p.sa[2] != 1 || p.sb[1] != 1) return false;
+    if (p.M > 64 || p.K % 8 != 0 || (p.M > 1 && p.sa[1] % 8 != 0) || (p.N > 1 && p.sb[2] % 8 != 0)) return false;
+    if (p.batch > 1 && (p.sa[0] % 8 != 0 || p.sb[0] % 8 != 0)) return false;
+    if (p.bh > 1 && (p.sa_h % 8 != 0 || p.sb_h % 8 != 0)) return false;
+    return true;
+}
+
+// Strips of columns, K chunks (whole stages) and their length.
+struct KringShape {
+    int strips, split, chunk;
+};
+
+KringShape kring_shape(const GemmArgs& p) {
+    KringShape r;
+    r.strips = (p.N + SKR_NB - 1) / SKR_NB;
+    const int stages = (p.K + SKR_KST - 1) / SKR_KST;
+    // (the fixup and the second launch read 16-byte rows of partials)
+    const int64_t want = p.N % 4 == 0 ? std::min<int64_t>(256 / ((int64_t)r.strips * p.batch), stages / 4) : 1;
+    const int per = want > 1 ? (int)((stages + want - 1) / want) : stages;
+    r.chunk = per * SKR_KST;
+    r.split = (stages + per - 1) / per;
+    return r;
+}
+
+template <int DT>
+void launch_kring(const GemmArgs& q, const KringShape& ks, hipStream_t s) {
+    const dim3 grid(ks.strips, q.split, q.batch), block(64 * SR_NW);
+    if (q.M <= 16) hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 1>), grid, block, 0, s, q);
+    else if (q.M <= 32) hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 2>), grid, block, 0, s, q);
+    else hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 4>), grid, block, 0, s, q);
+}
+
 bool ring_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
     if (b_kmajor || !vec) return false;
     auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
@@ -303,18 +483,50 @@ bool skinny_applies(int64_t M, int64_t N, int64_t K, int64_t batch) {
     return M >= 1 && M <= 16 && N >= 64 && K >= 64 && batch <= 65535;
 }
 
+bool skinny_wide_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
+    return p.M > 16 && p.M <= (p.K < 8192 ? 64 : 32) && skinny_applies(16, p.N, p.K, p.batch) && kring_applies(p, b_kmajor, vec);
+}
+
 const char* skinny_name(const GemmArgs& p, bool b_kmajor, bool vec) {
     if (ring_applies(p, b_kmajor, vec)) return ring_splits(p) > 1 ? "gemm16_skinny_ring_splitk" : "gemm16_skinny_ring";
     return b_kmajor ? "gemm16_skinny_bk" : "gemm16_skinny_bn";
 }
 
 size_t skinny_scratch_bytes(const GemmArgs& p, bool b_kmajor, bool vec) {
+    if (kring_applies(p, b_kmajor, vec)) {
+        const int split = kring_shape(p).split;
+        return split > 1 ? (size_t)split * p.batch * p.M * p.N * 4 : 0;
+    }
     if (!ring_applies(p, b_kmajor, vec)) return 0;
     const int split = ring_splits(p);
     return split > 1 ? (size_t)split * p.batch * p.M * p.N * 4 : 0;
 }
 
 hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, hipStream_t s, float* part) {
+    if (kring_applies(p, b_kmajor, vec)) {
+        GemmArgs q = p;
+        const KringShape ks = kring_shape(p);
+        q.split = ks.split;
+        q.k_chunk = ks.chunk;
+        Scratch scratch;
+        if (q.split > 1 && !part) {
+            // A call without scratch of its own (capture: its pool and counters must not be touched; no memory) runs
+            // unsplit, as this layout always did.
+            const bool can = scratch_usable(s) && (int64_t)q.split * p.batch * p.M * p.N * 4 < (int64_t(1) << 31);
+            q.part = can ? static_cast<float*>(scratch.get((size_t)q.split * p.batch * p.M * p.N * 4, s)) : nullptr;
+            if (q.part) q.tile_count = split_counters(s, (int64_t)ks.strips * p.batch);
+            else q.split = 1;
+        } else {
+            q.part = part;
+        }
+        if (dtype == TVK_F16) launch_kring<TVK_F16>(q, ks, s);
+        else launch_kring<TVK_BF16>(q, ks, s);
+        if (q.split > 1 && !q.tile_count) {
+            if (dtype == TVK_F16) launch_split_reduce<TVK_F16>(q, s);
+            else launch_split_reduce<TVK_BF16>(q, s);
+        }
+        return hipGetLastError();
+    }
     if (ring_applies(p, b_kmajor, vec)) {
         GemmArgs q = p;
         q.split = ring_splits(p);
@@ -341,10 +553,10 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
     dim3 grid(strips, 1, p.batch);
 #define TVK_SK(D, BKM, V) hipLaunchKernelGGL((gemm_skinny_kernel<D, BKM, V>), grid, dim3(64 * SK_NW), 0, s, p)
     if (dtype == TVK_F16) {
-        if (b_kmajor) { if (vec) TVK_SK(TVK_F16, true, true); else TVK_SK(TVK_F16, true, false); }
+        if (b_kmajor) TVK_SK(TVK_F16, true, false);   // (with 16-byte rows: the ring)
         else { if (vec) TVK_SK(TVK_F16, false, true); else TVK_SK(TVK_F16, false, false); }
     } else {
-        if (b_kmajor) { if (vec) TVK_SK(TVK_BF16, true, true); else TVK_SK(TVK_BF16, true, false); }
+        if (b_kmajor) TVK_SK(TVK_BF16, true, false);
         else { if (vec) TVK_SK(TVK_BF16, false, true); else TVK_SK(TVK_BF16, false, false); }
     }
 #undef TVK_SK

@@ -146,6 +146,14 @@ void* Scratch::get(size_t bytes, hipStream_t stream) {
     return buf->ptr;
 }
 
+bool scratch_usable(hipStream_t stream) {
+    if (stream == hipStreamPerThread) return false;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 void Scratch::release() {
     if (!lease_) return;
     device_scratch(device_)->pool.release(static_cast<ScratchPool<HipScratchBackend>::Buffer*>(lease_));

@@ -56,6 +56,13 @@ private:
     hipStream_t stream_ = nullptr;
 };
 
+// Whether a call that can do without may lease scratch for kernels on
+// `stream`: not while the stream is captured (a graph may be replayed on
+// another stream, where the pool's ownership by stream does not hold, and
+// capture must not allocate), nor on hipStreamPerThread, a handle that stands
+// for a stream of each thread.
+bool scratch_usable(hipStream_t stream);
+
 // Split-K tile counters for kernels queued on `stream` of the current device:
 // `count` words, zero now and left zero by every kernel that uses them (the
 // last workgroup of a tile resets its counter). One array per stream, so
