@@ -176,11 +176,12 @@ __global__ __launch_bounds__(128 * WGN) void gemm16_mfma_kernel(GemmArgs p) {
     tile_of(blockIdx.x, p.tiles_m * p.tiles_n, p.tiles_m, p.tiles_n, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
 
+    constexpr bool SPLIT = BM == 128 && BN == 128;   // the only tiles whose launches split K
     // operand buffers of this batch (and of this k split): A rows are M, B rows are N
     const uint16_t* A = reinterpret_cast<const uint16_t*>(p.a) + a_boff(p, b);
     const uint16_t* B = reinterpret_cast<const uint16_t*>(p.b) + b_boff(p, b);
     int K = p.K;
-    if (p.split > 1) {
+    if (SPLIT && p.split > 1) {
         const int kb = blockIdx.z * p.k_chunk;
         A += (int64_t)kb * p.sa[2];
         B += (int64_t)kb * p.sb[1];
@@ -283,8 +284,8 @@ __global__ __launch_bounds__(128 * WGN) void gemm16_mfma_kernel(GemmArgs p) {
 
     // accumulator layout of v_mfma_f32_32x32x16: lane holds column lane%32,
     // register r holds row (r/4)*8 + (lane/32)*4 + r%4
-    if (p.split > 1) {
-        float* part = p.part + ((int64_t)blockIdx.z * p.batch + b) * p.M * p.N;
+    if (SPLIT && p.split > 1) {
+        float* part = p.part + ((int64_t)blockIdx.z * p.batch + b) * p.M * p.np;
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(128 * WGN) void gemm16_mfma_kernel(GemmArgs p) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int row = row0 + (r / 4) * 8 + (r % 4);
-                    if (row < p.M) part[(int64_t)row * p.N + col] = acc[i][j][r];
+                    if (row < p.M) part[(int64_t)row * p.np + col] = acc[i][j][r];
                 }
             }
         return;
@@ -611,26 +612,47 @@ __global__ __launch_bounds__(256) void gemm_seq16_kernel(GemmArgs p) {
 
 // ----------------------------------------------------------------------------
 // operand repack: dst[b][r][c] = src(b, r, c) for c < C, 0 for C <= c < Cp
-// (c is the operand's contiguous dimension; rows are Cp elements apart)
+// (c is the operand's contiguous dimension; rows are Cp elements apart), of
+// one or both operands of a product in one launch. A thread moves 8 elements
+// with one 16-byte load of any alignment (the last chunk of a row goes element
+// by element): bound by its launch, 5.8 us in the trace for either operand of
+// 1000 x 777 x 3000 and for both (two launches of 5.3 before).
 // ----------------------------------------------------------------------------
 
-__global__ __launch_bounds__(256) void repack16_kernel(const uint16_t* src, uint16_t* dst, int64_t s0, int64_t sr, int64_t sc,
-                                                        int batch, int R, int C, int Cp) {
-    const int64_t chunks = (int64_t)batch * R * (Cp / 8);
-    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < chunks; q += (int64_t)gridDim.x * 256) {
-        const int c0 = (int)(q % (Cp / 8)) * 8;
-        const int64_t br = q / (Cp / 8);
-        const int r = (int)(br % R), b = (int)(br / R);
-        const uint16_t* sp = src + (int64_t)b * s0 + (int64_t)r * sr;
-        uint32_t w[4];
+struct RepackArgs {
+    const uint16_t* src;
+    uint16_t* dst;
+    int64_t s0, sr;   // batch and row strides of src
+    int R, C, Cp;
+    int64_t chunks;   // 8-element chunks of dst, 0: none
+};
+struct RepackPair {
+    RepackArgs op[2];
+};
+
+__global__ __launch_bounds__(256) void repack16_kernel(RepackPair pair) {
+    const int64_t total = pair.op[0].chunks + pair.op[1].chunks;
+    for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < total; t += (int64_t)gridDim.x * 256) {
+        const bool second = t >= pair.op[0].chunks;
+        const RepackArgs& a = pair.op[second ? 1 : 0];
+        const int64_t q = second ? t - pair.op[0].chunks : t;
+        const int c0 = (int)(q % (a.Cp / 8)) * 8;
+        const int64_t br = q / (a.Cp / 8);
+        const int r = (int)(br % a.R), b = (int)(br / a.R);
+        const uint16_t* sp = a.src + (int64_t)b * a.s0 + (int64_t)r * a.sr + c0;
+        u32x4 w;
+        if (c0 + 8 <= a.C) {
+            __builtin_memcpy(&w, sp, 16);
+        } else {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int c = c0 + 2 * e;
-            const uint32_t lo = c < C ? sp[(int64_t)c * sc] : 0u;
-            const uint32_t hi = c + 1 < C ? sp[(int64_t)(c + 1) * sc] : 0u;
-            w[e] = lo | (hi << 16);
+            for (int e = 0; e < 4; ++e) {
+                const int c = c0 + 2 * e;
+                const uint32_t lo = c < a.C ? sp[2 * e] : 0u;
+                const uint32_t hi = c + 1 < a.C ? sp[2 * e + 1] : 0u;
+                w[e] = lo | (hi << 16);
+            }
         }
-        *reinterpret_cast<u32x4*>(dst + ((int64_t)b * R + r) * Cp + c0) = u32x4{w[0], w[1], w[2], w[3]};
+        *reinterpret_cast<u32x4*>(a.dst + ((int64_t)b * a.R + r) * a.Cp + c0) = w;
     }
 }
 
@@ -684,6 +706,7 @@ GemmArgs make_args(const tvk_gemm_desc& d) {
         p.sa[i] = d.a_stride[i]; p.sb[i] = d.b_stride[i]; p.sbias[i] = d.bias_stride[i]; p.sc[i] = d.c_stride[i];
     }
     p.M = (int)d.M; p.N = (int)d.N; p.K = (int)d.K;
+    p.np = p.N;
     p.batch = (int)d.batch;
     p.alpha = (float)d.alpha;
     p.beta = (float)d.beta;
@@ -702,11 +725,17 @@ GemmArgs make_args(const tvk_gemm_desc& d) {
 int64_t pad8(int64_t v) { return (v + 7) / 8 * 8; }
 int64_t repack_ld(int64_t v, bool kdim) { return kdim ? (v + 31) / 32 * 32 : pad8(v); }
 
+// Elements between rows of float32 partials: whole 16-byte groups (the
+// allocation-free entry point, whose scratch is fixed, keeps rows of N).
+int64_t part_pitch(int64_t n) { return (n + 3) / 4 * 4; }
+
 // Whether every load of k in [K, K rounded up to 32) returns zero under plan
-// pl: each k-contiguous operand is repacked (zero-padded rows), and each
-// m/n-contiguous one has rows at least as long as its extent, so row K and
-// beyond lie past its buffer range.
+// pl: each k-contiguous operand is repacked (zero-padded rows) or ends on a
+// whole 16-byte chunk (k_masked), and each m/n-contiguous one has rows at
+// least as long as its extent, so row K and beyond lie past its buffer range.
 bool k_tail_zero(const tvk_gemm_desc& d, const struct Plan& pl);
+// Whether the ring has to mask a k-contiguous operand's chunks past K.
+bool k_masked(const tvk_gemm_desc& d, const struct Plan& pl);
 
 // Arguments as the kernels see them once the planned repacks are done (the
 // pointers of repacked operands only matter for alignment: workspace offsets
@@ -811,6 +840,30 @@ bool split_plan(const tvk_gemm_desc& d, int64_t want, Plan& pl, Kern kern = Kern
     return true;
 }
 
+// 256x256 tiles whose last round on the 256 CUs is at most half full, with
+// few rounds (the transformer's gate_up, 8192x3072x512: 384 tiles, one and
+// a half rounds; 6144^3: 576 tiles): 128x256 tiles, twice as many, whole
+// rounds (gate_up 38.2-40.7 us against 41.9-45.8 for 256x256; 6144^3 409
+// against 449 for 256x128 tiles)
+bool half_round(int64_t t256) { return t256 < 1024 && t256 % 256 != 0 && t256 % 256 <= 128; }
+
+// The ring tile of a product too small for whole rounds of 256x256 tiles: with
+// more than one round of 128x128 tiles at K >= 1024 the tile whose rounds of
+// 256 workgroups cost least, a 128x128 / 128x256 / 256x256 tile costing 1 :
+// 1.6 : 2.4 (measured at 2560^3, 3072^3, 4096x2048x4096 and 2048x4096x2048:
+// 1.10-1.24x over 128x128 tiles)
+Kern medium_tile(const tvk_gemm_desc& d) {
+    const int64_t t128 = ((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
+    if (t128 <= 256 || d.K < 1024) return Kern::DMA128;
+    const int64_t t12 = ((d.M + 127) / 128) * ((d.N + 255) / 256) * d.batch;
+    const int64_t t256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * d.batch;
+    auto rounds = [](int64_t t) { return (double)((t + 255) / 256); };
+    const double c128 = rounds(t128), c12 = 1.6 * rounds(t12), c256 = 2.4 * rounds(t256);
+    if (c256 < c128 && c256 < c12 && d.M >= 256 && d.N >= 256) return Kern::DMA256;
+    if (c12 < c128 && d.N >= 256) return Kern::DMA128X256;
+    return Kern::DMA128;
+}
+
 // The kernel chosen from the shape alone (used unless the kernel-choice table
 // holds another candidate for the product's shape class).
 Plan make_plan(const tvk_gemm_desc& d) {
@@ -839,15 +892,10 @@ Plan make_plan(const tvk_gemm_desc& d) {
         return pl;
     }
     const bool dma_ok = pl.vec && dma_applies(repacked_args(d, pl), pl.ak, pl.bk);
-    // 256x256 tiles whose last round on the 256 CUs is at most half full, with
-    // few rounds (the transformer's gate_up, 8192x3072x512: 384 tiles, one and
-    // a half rounds; 6144^3: 576 tiles): 128x256 tiles, twice as many, whole
-    // rounds (gate_up 38.2-40.7 us against 41.9-45.8 for 256x256; 6144^3 409
-    // against 449 for 256x128 tiles)
-    const bool half_round = t256 < 1024 && t256 % 256 != 0 && t256 % 256 <= 128;
     if (big && dma_ok) {
-        pl.kern = half_round ? Kern::DMA128X256 : Kern::DMA256;
-        pl.name = half_round ? "gemm16_dma_128x256" : "gemm16_dma_256x256";
+        const bool half = half_round(t256);
+        pl.kern = half ? Kern::DMA128X256 : Kern::DMA256;
+        pl.name = half ? "gemm16_dma_128x256" : "gemm16_dma_256x256";
     } else if (big) {
         // 8 waves; the 4-wave form stays a kernel-choice candidate
         pl.kern = Kern::MFMA256W8;
@@ -885,25 +933,41 @@ Plan make_plan(const tvk_gemm_desc& d) {
             // register-staged one on 8192 x {512, 256} x 512)
             pl.kern = Kern::DMA128;
             pl.name = "gemm16_dma_128x128";
-            // More than one round of 128x128 tiles at K >= 1024: the tile whose
-            // rounds of 256 workgroups cost least, a 128x128 / 128x256 / 256x256
-            // tile costing 1 : 1.6 : 2.4 (measured at 2560^3, 3072^3, 4096x2048x4096
-            // and 2048x4096x2048: 1.10-1.24x over 128x128 tiles)
-            if (t128 > 256 && d.K >= 1024) {
-                const int64_t t12 = ((d.M + 127) / 128) * ((d.N + 255) / 256) * d.batch;
-                auto rounds = [](int64_t t) { return (double)((t + 255) / 256); };
-                const double c128 = rounds(t128), c12 = 1.6 * rounds(t12), c256 = 2.4 * rounds(t256);
-                if (c256 < c128 && c256 < c12 && d.M >= 256 && d.N >= 256) {
-                    pl.kern = Kern::DMA256;
-                    pl.name = "gemm16_dma_256x256";
-                } else if (c12 < c128 && d.N >= 256) {
-                    pl.kern = Kern::DMA128X256;
-                    pl.name = "gemm16_dma_128x256";
-                }
-            }
+            pl.kern = medium_tile(d);
+            if (pl.kern == Kern::DMA256) pl.name = "gemm16_dma_256x256";
+            else if (pl.kern == Kern::DMA128X256) pl.name = "gemm16_dma_128x256";
         }
     }
     return pl;
+}
+
+// The ring tile of a product that runs the register-staged plan's name but
+// whose operands the ring can read with its edge cases (K off the 32 grid with
+// 16-byte rows, or m/n-contiguous rows repacked to whole 16-byte chunks); false
+// when the register-staged kernel itself runs. The names stay those of "any K":
+// they are what the kernel-choice table and its files record.
+//   256x256: the register-staged 8-wave kernel spills (float16 5000^3 row-major
+//     4271 us, 249 here; k-contiguous 4224 and 309; 6001 x 6003 x 6005 7070 and
+//     478), so the ring always.
+//   128x128: 2000^3 43.3 -> 23.7 us, 4100 x 1037 x 4100 110 -> 69, 2048 x 3000
+//     x 904 24.4 -> 21.7. Two k-contiguous operands read half lines a stage:
+//     ahead from K = 1024 without a split (2000^3 33.8 -> 27.7), behind below
+//     (2048 x 3000 x 904 22.8 against 24.4) and split (333 x 777 x 5000 20.8
+//     against 22.9).
+bool edge_ring(const tvk_gemm_desc& d, const Plan& pl, int& tile) {
+    if ((pl.kern != Kern::MFMA256W8 && pl.kern != Kern::MFMA128) || !pl.vec) return false;
+    if (pl.kern == Kern::MFMA128 && pl.ak && pl.bk && (pl.split > 1 || d.K < 1024)) return false;
+    const GemmArgs p = repacked_args(d, pl);
+    if (dma_applies(p, pl.ak, pl.bk) || !dma_applies(p, pl.ak, pl.bk, true)) return false;
+    const int64_t t256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * d.batch;
+    if (pl.kern == Kern::MFMA256W8) tile = half_round(t256) ? DMA_TILE_128X256 : 256;
+    else if (pl.split > 1) tile = 128;
+    else switch (medium_tile(d)) {
+        case Kern::DMA256: tile = 256; break;
+        case Kern::DMA128X256: tile = DMA_TILE_128X256; break;
+        default: tile = 128; break;
+    }
+    return true;
 }
 
 // A candidate's name in the kernel-choice table: the kernel name, and the
@@ -1008,14 +1072,19 @@ GemmArgs repacked_args(const tvk_gemm_desc& d, const Plan& pl) {
         p.b_ext = 2 * p.sb[0];
     }
     p.kzero = k_tail_zero(d, pl) ? 1 : 0;
+    p.kmask = k_masked(d, pl) ? 1 : 0;
     return p;
 }
 
 bool k_tail_zero(const tvk_gemm_desc& d, const Plan& pl) {
     if (d.K % 32 == 0) return true;
-    const bool a_ok = pl.ak ? pl.repack_a : (pl.repack_a || d.a_stride[2] >= d.M);
-    const bool b_ok = pl.bk ? pl.repack_b : (pl.repack_b || d.b_stride[1] >= d.N);
+    const bool a_ok = pl.ak ? (pl.repack_a || d.K % 8 == 0) : (pl.repack_a || d.a_stride[2] >= d.M);
+    const bool b_ok = pl.bk ? (pl.repack_b || d.K % 8 == 0) : (pl.repack_b || d.b_stride[1] >= d.N);
     return a_ok && b_ok;
+}
+
+bool k_masked(const tvk_gemm_desc& d, const Plan& pl) {
+    return d.K % 32 != 0 && ((pl.ak && !pl.repack_a) || (pl.bk && !pl.repack_b));
 }
 
 #define TVK_LAYOUT_SWITCH(PL, NTHR, KERNEL, ...)                                            \
@@ -1052,14 +1121,14 @@ void launch_seq16(const Plan& pl, GemmArgs& p, dim3 grid, hipStream_t s) {
 // Scratch bytes one batch chunk of `nb` matrices needs under plan pl:
 // repacked operands (256-byte aligned each), then split-K partials, or the
 // streaming kernel's partials. rep_a / rep_b / part_b return the pieces.
-size_t plan_scratch_bytes(const tvk_gemm_desc& d, const Plan& pl, int nb, size_t* rep_a_out = nullptr,
+size_t plan_scratch_bytes(const tvk_gemm_desc& d, const Plan& pl, int nb, bool fixed, size_t* rep_a_out = nullptr,
                           size_t* rep_b_out = nullptr) {
     auto al256 = [](size_t v) { return (v + 255) / 256 * 256; };
     const int64_t a_rows = pl.ak ? d.M : d.K, a_ld = repack_ld(pl.ak ? d.K : d.M, pl.ak);
     const int64_t b_rows = pl.bk ? d.N : d.K, b_ld = repack_ld(pl.bk ? d.K : d.N, pl.bk);
     const size_t rep_a = pl.repack_a ? al256((size_t)nb * a_rows * a_ld * 2) : 0;
     const size_t rep_b = pl.repack_b ? al256((size_t)nb * b_rows * b_ld * 2) : 0;
-    size_t part_b = pl.split > 1 ? (size_t)pl.split * nb * d.M * d.N * 4 : 0;
+    size_t part_b = pl.split > 1 ? (size_t)pl.split * nb * d.M * (fixed ? d.N : part_pitch(d.N)) * 4 : 0;
     if (pl.kern == Kern::SKINNY) {
         GemmArgs q = make_args(d);
         q.batch = nb;
@@ -1093,7 +1162,7 @@ tvk_status run(const tvk_gemm_desc& d, const Plan& pl, hipStream_t s, char* fixe
         const int64_t a_rows = pl.ak ? d.M : d.K, a_ld = repack_ld(pl.ak ? d.K : d.M, pl.ak);
         const int64_t b_rows = pl.bk ? d.N : d.K, b_ld = repack_ld(pl.bk ? d.K : d.N, pl.bk);
         size_t rep_a = 0, rep_b = 0;
-        size_t need = plan_scratch_bytes(d, pl, nb, &rep_a, &rep_b);
+        size_t need = plan_scratch_bytes(d, pl, nb, fixed != nullptr, &rep_a, &rep_b);
         if (pl.kern == Kern::SKINNY && !fixed) need = 0;   // launch_skinny leases its own
         char* ws = nullptr;
         Scratch scratch;
@@ -1106,15 +1175,14 @@ tvk_status run(const tvk_gemm_desc& d, const Plan& pl, hipStream_t s, char* fixe
             if (!ws) return fail(TVK_ERR_OOM, "tvk_gemm: no workspace for repacked operands or split-K partials");
         }
         if constexpr (DT != TVK_F32) {
-            auto repack = [&](const void* src, int64_t s0, int64_t sr, int64_t sc, int64_t rows, int64_t cols, int64_t ld, char* dst) {
-                const int64_t chunks = (int64_t)nb * rows * (ld / 8);
-                const unsigned blocks = (unsigned)std::min<int64_t>((chunks + 255) / 256, 16384);
-                hipLaunchKernelGGL(repack16_kernel, dim3(blocks), dim3(256), 0, s, static_cast<const uint16_t*>(src),
-                                   reinterpret_cast<uint16_t*>(dst), s0, sr, sc, nb, (int)rows, (int)cols, (int)ld);
+            RepackPair pair{};
+            auto repack = [&](RepackArgs& r, const void* src, int64_t s0, int64_t sr, int64_t rows, int64_t cols, int64_t ld, char* dst) {
+                r = RepackArgs{static_cast<const uint16_t*>(src), reinterpret_cast<uint16_t*>(dst), s0, sr, (int)rows, (int)cols, (int)ld,
+                               (int64_t)nb * rows * (ld / 8)};
             };
             if (pl.repack_a) {
-                if (pl.ak) repack(q.a, d.a_stride[0], d.a_stride[1], d.a_stride[2], d.M, d.K, a_ld, ws);
-                else repack(q.a, d.a_stride[0], d.a_stride[2], d.a_stride[1], d.K, d.M, a_ld, ws);
+                if (pl.ak) repack(pair.op[0], q.a, d.a_stride[0], d.a_stride[1], d.M, d.K, a_ld, ws);
+                else repack(pair.op[0], q.a, d.a_stride[0], d.a_stride[2], d.K, d.M, a_ld, ws);
                 q.a = ws;
                 q.sa[0] = a_rows * a_ld;
                 q.sa[1] = pl.ak ? a_ld : 1;
@@ -1122,14 +1190,33 @@ tvk_status run(const tvk_gemm_desc& d, const Plan& pl, hipStream_t s, char* fixe
                 q.a_ext = 2 * q.sa[0];
             }
             if (pl.repack_b) {
-                if (pl.bk) repack(q.b, d.b_stride[0], d.b_stride[2], d.b_stride[1], d.N, d.K, b_ld, ws + rep_a);
-                else repack(q.b, d.b_stride[0], d.b_stride[1], d.b_stride[2], d.K, d.N, b_ld, ws + rep_a);
+                if (pl.bk) repack(pair.op[1], q.b, d.b_stride[0], d.b_stride[2], d.N, d.K, b_ld, ws + rep_a);
+                else repack(pair.op[1], q.b, d.b_stride[0], d.b_stride[1], d.K, d.N, b_ld, ws + rep_a);
                 q.b = ws + rep_a;
                 q.sb[0] = b_rows * b_ld;
                 q.sb[1] = pl.bk ? 1 : b_ld;
                 q.sb[2] = pl.bk ? b_ld : 1;
                 q.b_ext = 2 * q.sb[0];
             }
+            if (pl.repack_a || pl.repack_b) {
+                const int64_t chunks = pair.op[0].chunks + pair.op[1].chunks;
+                const unsigned blocks = (unsigned)std::min<int64_t>((chunks + 255) / 256, 16384);
+                hipLaunchKernelGGL(repack16_kernel, dim3(blocks), dim3(256), 0, s, pair);
+            }
+            q.kmask = k_masked(d, pl) ? 1 : 0;
+            if (!fixed) q.np = (int)part_pitch(d.N);
+        }
+        int tile = 0;
+        if constexpr (DT != TVK_F32) if (edge_ring(d, pl, tile)) {
+            if (pl.split > 1) {
+                q.part = reinterpret_cast<float*>(ws + rep_a + rep_b);
+                q.split = pl.split;
+                q.k_chunk = pl.k_chunk;
+            }
+            const hipError_t e = launch_dma(DT, q, pl.ak, pl.bk, tile, s, 4);
+            if (e != hipSuccess) return fail(TVK_ERR_DEVICE, std::string("tvk_gemm: launch failed: ") + hipGetErrorString(e));
+            if (pl.split > 1) launch_split_reduce<DT>(q, s);
+            continue;
         }
         switch (pl.kern) {
         case Kern::K0: {
@@ -1450,7 +1537,7 @@ extern "C" tvk_status tvk_gemm_noalloc(const tvk_gemm_desc* desc) {
         first.N = nc;
     }
     const int nb = (int)std::min<int64_t>(65535, d.batch);
-    const size_t need = plan_scratch_bytes(first, make_plan(first), nb);
+    const size_t need = plan_scratch_bytes(first, make_plan(first), nb, true);
     if (need > kNoAllocScratch)
         return fail(TVK_ERR_INVALID, "tvk_gemm_noalloc: this product needs " + std::to_string(need) +
                                          " bytes of scratch (split-K partials or repacked operands), more than the " +

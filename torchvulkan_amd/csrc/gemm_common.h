@@ -19,15 +19,16 @@ struct GemmArgs {
     int act;
     int tiles_m, tiles_n;
     // split-K (split > 1): blockIdx.z takes k in [z*k_chunk, (z+1)*k_chunk) and
-    // writes float32 partials to part[z][batch][M][N]; a second kernel sums
-    // them in z order and applies the epilogue
+    // writes float32 partials to part[z][batch][M][np]; a second kernel sums
+    // them in z order and applies the epilogue. np: N, or N rounded up to 4
+    // (16-byte rows of partials)
     float* part;
     int k_chunk;
     int split;
     // 1: loads of k in [K, K rounded up to 32) return zeros for both operands
-    // (a k-contiguous operand was copied with zero-padded rows; rows past K of
-    // an m/n-contiguous one lie outside its buffer range), so the LDS-ring
-    // kernels may run the last k step whole
+    // (a k-contiguous operand was copied with zero-padded rows, or kmask;
+    // rows past K of an m/n-contiguous one lie outside its buffer range), so
+    // the LDS-ring kernels may run the last k step whole
     int kzero;
     // bytes of one matrix of a repacked operand (the whole zero-padded
     // [rows][ld] copy, which the LDS-ring kernels' buffer ranges then cover);
@@ -41,6 +42,10 @@ struct GemmArgs {
     // addressed with stride [0] and the *_h stride (batch_off)
     int bh;
     int64_t sa_h, sb_h, sbias_h, sc_h;
+    int np;      // elements between rows of partials
+    // 1: a k-contiguous operand's 16-byte chunks past K (a multiple of 8) are
+    // the next row's values: the ring loads zeros for them in the last k step
+    int kmask;
 };
 
 // Element offset of batch b of an operand with outer stride s0 and inner
@@ -183,9 +188,14 @@ __device__ inline void tile_of(int bid, int nblocks, int tiles_m, int tiles_n, i
     tn = in / gm;
 }
 
-// Finishes four consecutive outputs (row, col .. col + 3) of matrix b from
-// their float32 sums: the epilogue, one rounding to the output type, and one
-// 8-byte store where the output rows are contiguous and 8-byte aligned (vec).
+// Vector stores to rows of any alignment (global memory takes them; a row of
+// 777 16-bit elements starts 16-byte aligned once in eight).
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2u __attribute__((ext_vector_type(2), aligned(2)));
+
+// Finishes four consecutive outputs (row, col .. col + 3; those below N) of
+// matrix b from their float32 sums: the epilogue, one rounding to the output
+// type, and one 8-byte store where the output rows are contiguous (vec).
 template <int DT>
 __device__ __forceinline__ void finish4(const GemmArgs& p, int b, int row, int col, f32x4 v, bool vec) {
     typedef typename elem<DT>::T T;
@@ -197,23 +207,21 @@ __device__ __forceinline__ void finish4(const GemmArgs& p, int b, int row, int c
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         float bv = 0.0f;
-        if (p.has_bias) bv = elem<DT>::to_f32(bp[(int64_t)r * p.sbias[2]]);
+        if (p.has_bias && col + r < p.N) bv = elem<DT>::to_f32(bp[(int64_t)r * p.sbias[2]]);
         h[r] = __builtin_bit_cast(uint16_t, elem<DT>::from_f32(epilogue(v[r], p.alpha, p.has_bias, bv, p.beta, p.act)));
     }
     T* cp = c + c_boff(p, b) + (int64_t)row * p.sc[1] + (int64_t)col * p.sc[2];
-    if (vec) {
-        st_nt(reinterpret_cast<u32x2*>(cp), u32x2{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)});
+    if (vec && col + 4 <= p.N) {
+        st_nt(reinterpret_cast<u32x2u*>(cp), u32x2u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16)});
     } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) cp[(int64_t)r * p.sc[2]] = __builtin_bit_cast(T, h[r]);
+        for (int r = 0; r < 4; ++r)
+            if (col + r < p.N) cp[(int64_t)r * p.sc[2]] = __builtin_bit_cast(T, h[r]);
     }
 }
 
 // Whether finish4 may store four outputs as one 8-byte write.
-__device__ __forceinline__ bool finish4_vec(const GemmArgs& p) {
-    return p.sc[2] == 1 && p.sc[1] % 4 == 0 && (p.batch == 1 || (p.sc[0] % 4 == 0 && (p.bh <= 1 || p.sc_h % 4 == 0))) &&
-           (reinterpret_cast<uintptr_t>(p.c) & 7) == 0;
-}
+__device__ __forceinline__ bool finish4_vec(const GemmArgs& p) { return p.sc[2] == 1; }
 
 // Split-K without a second launch. The float32 partial planes of such a
 // launch are written through to memory and read back coherently, without a
@@ -304,11 +312,12 @@ namespace {
 // epilogue and rounds once to the output type.
 template <int DT>
 __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmArgs p) {
-    const int64_t mn = (int64_t)p.M * p.N;
+    const int64_t mn = (int64_t)p.M * p.np;
     const int64_t total = (int64_t)p.batch * mn;
     for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (int64_t)gridDim.x * 256) {
         const int b = (int)(idx / mn);
         const int64_t e = idx - (int64_t)b * mn;
+        if (p.np != p.N && (int)(e % p.np) >= p.N) continue;
         float v = p.part[idx];
         // eight planes' loads in flight before their adds (still in split order)
         int z = 1;
@@ -330,17 +339,17 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmArgs p) {
             for (int u = 0; u < 7; ++u)
                 if (u < rem) v += w[u];
         }
-        store_out<DT>(p, b, (int)(e / p.N), (int)(e % p.N), v);
+        store_out<DT>(p, b, (int)(e / p.np), (int)(e % p.np), v);
     }
 }
 
-// The same sum, four consecutive outputs of one row a thread (N % 4 == 0, so
+// The same sum, four consecutive outputs of one row a thread (np % 4 == 0, so
 // a group never straddles two rows): 16-byte loads from each partial plane,
 // added in split order, the epilogue inline, and one 8-byte store where the
-// output rows are contiguous and 8-byte aligned (VEC).
+// output rows are contiguous (VEC).
 template <int DT, bool VEC>
 __global__ __launch_bounds__(256) void gemm_split_reduce4_kernel(GemmArgs p) {
-    const int64_t mn = (int64_t)p.M * p.N;
+    const int64_t mn = (int64_t)p.M * p.np;
     const int64_t total = (int64_t)p.batch * mn;
     const int64_t groups = total / 4;
     for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < groups; q += (int64_t)gridDim.x * 256) {
@@ -370,7 +379,7 @@ __global__ __launch_bounds__(256) void gemm_split_reduce4_kernel(GemmArgs p) {
         }
         const int b = (int)(idx / mn);
         const int64_t e = idx - (int64_t)b * mn;
-        const int row = (int)(e / p.N), col = (int)(e - (int64_t)row * p.N);
+        const int row = (int)(e / p.np), col = (int)(e - (int64_t)row * p.np);
         finish4<DT>(p, b, row, col, v, VEC);
     }
 }
@@ -378,16 +387,15 @@ __global__ __launch_bounds__(256) void gemm_split_reduce4_kernel(GemmArgs p) {
 }  // namespace
 
 // The split-K reduction for a float16/bfloat16 output: the four-wide kernel
-// where N is a multiple of 4 and the output fills at least 256 of its
+// where partial rows are a multiple of 4 and the output fills at least 256 of its
 // workgroups or there are 8 or more partial planes (smaller outputs of few
 // planes, such as the M <= 16 products', keep more workgroups with one output
 // a thread: measured 0.2 us faster there).
 template <int DT>
 inline void launch_split_reduce(const GemmArgs& q, hipStream_t s) {
-    const int64_t total = (int64_t)q.batch * q.M * q.N;
-    if (q.N % 4 == 0 && (total >= 4 * 256 * 256 || q.split >= 8)) {
-        const bool vec = q.sc[2] == 1 && q.sc[1] % 4 == 0 && (q.batch == 1 || (q.sc[0] % 4 == 0 && (q.bh <= 1 || q.sc_h % 4 == 0))) &&
-                         (reinterpret_cast<uintptr_t>(q.c) & 7) == 0;
+    const int64_t total = (int64_t)q.batch * q.M * q.np;
+    if (q.np % 4 == 0 && (total >= 4 * 256 * 256 || q.split >= 8)) {
+        const bool vec = q.sc[2] == 1;
         const unsigned blocks = (unsigned)std::min<int64_t>((total / 4 + 255) / 256, 8192);
         if (vec) hipLaunchKernelGGL((gemm_split_reduce4_kernel<DT, true>), dim3(blocks), dim3(256), 0, s, q);
         else hipLaunchKernelGGL((gemm_split_reduce4_kernel<DT, false>), dim3(blocks), dim3(256), 0, s, q);
@@ -432,7 +440,9 @@ __device__ inline u32x4 load_chunk(__amdgpu_buffer_rsrc_t r, bool row_ok, int64_
 // Tile kernel with operands fetched straight into LDS (gemm_dma.hip).
 // dma_applies: the operands meet its alignment and K granularity; launch_dma
 // returns hipSuccess or the launch error.
-bool dma_applies(const GemmArgs& p, bool a_kmajor, bool b_kmajor);
+// edges: also the products whose last k step needs masks (kmask) or whose
+// m/n-contiguous rows end inside a 16-byte chunk of a repacked operand.
+bool dma_applies(const GemmArgs& p, bool a_kmajor, bool b_kmajor, bool edges = false);
 // tile: 256 (256x256), 128 (128x128), DMA_TILE_128X256 or DMA_TILE_256X128
 constexpr int DMA_TILE_128X256 = 1, DMA_TILE_256X128 = 2;
 hipError_t launch_dma(int dtype, GemmArgs& p, bool a_kmajor, bool b_kmajor, int tile, hipStream_t s, int stages = 4);

@@ -108,8 +108,9 @@ template <bool KM, int D, int W, bool XS>
 struct DmaSrc {
     static_assert(KM || W >= 128, "the MN swizzle moves chunks within 16-chunk blocks");
     uint32_t off[D];
-    uint32_t kstep;   // bytes per stage along k
-    __device__ inline void init(int64_t s_row, int64_t s_k, int row0, int rows, int wave, int lane) {
+    uint32_t tail[D];   // added in the last stage: past the buffer for a KM chunk at or past k_left, else 0
+    uint32_t kstep;     // bytes per stage along k
+    __device__ inline void init(int64_t s_row, int64_t s_k, int row0, int rows, int wave, int lane, int k_left) {
         constexpr int CPR = 2 * W / 16;   // 16-byte chunks per MN k-row
 #pragma unroll
         for (int i = 0; i < D; ++i) {
@@ -119,11 +120,13 @@ struct DmaSrc {
                 const int c = (lane % 4) ^ swz_km<XS>(row);
                 const int gr = row0 + row;
                 off[i] = gr < rows ? (uint32_t)(((int64_t)gr * s_row + c * 8) * 2) : kOOB;
+                tail[i] = c * 8 >= k_left && gr < rows ? kOOB : 0;
             } else {
                 const int kr = blk * (64 / CPR) + lane / CPR;
                 const int c = (lane % CPR) ^ swz_mn<XS>(kr);
                 const int gc = row0 + c * 8;
                 off[i] = gc < rows ? (uint32_t)(((int64_t)kr * s_k + gc) * 2) : kOOB;
+                tail[i] = 0;
             }
         }
         kstep = KM ? (uint32_t)(D_BK * 2) : (uint32_t)(D_BK * s_k * 2);
@@ -171,7 +174,8 @@ constexpr int dma_threads(int bm, int bn) { return 64 * ((bm == 256 && bn == 256
 // lookahead to cover memory latency: short K, one workgroup per CU).
 // BL: C-in staged through the ring (256x256 tiles with a bias; a variant of
 // its own because the bias loads' offsets cost the k loop registers).
-template <int DT, bool AK, bool BK, int BM, int BN, int NS, bool BL = false>
+// KT: the last k step masks a k-contiguous operand's chunks past K (kmask).
+template <int DT, bool AK, bool BK, int BM, int BN, int NS, bool BL = false, bool KT = false>
 __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArgs p) {
     constexpr int D_NS = NS;
     typedef DCfg<BM, BN> G;
@@ -196,8 +200,10 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
     constexpr bool XS = !G::BIG;   // the wide (conflict-free) swizzles
     DmaSrc<AK, G::DA, BM, XS> da;
     DmaSrc<BK, G::DB, BN, XS> db;
-    da.init(p.sa[1], p.sa[2], m0, p.M, wave, lane);
-    db.init(p.sb[2], p.sb[1], n0, p.N, wave, lane);
+    const int k_left = p.K % D_BK;   // (KT only)
+    da.init(p.sa[1], p.sa[2], m0, p.M, wave, lane, k_left);
+    db.init(p.sb[2], p.sb[1], n0, p.N, wave, lane, k_left);
+    const uint32_t k_last = (uint32_t)(p.K / D_BK);   // the stage that holds K's end
     // split-K (grid z): this workgroup's k range starts at stage kt0
     const int kt0 = p.split > 1 ? (int)blockIdx.z * (p.k_chunk / D_BK) : 0;
     // (a K off the 32 grid runs its last step whole: split chunks are whole
@@ -237,8 +243,11 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                 return;
             }
         }
-        if (q < G::DA) dma16(live ? ra : ra_none, slot + (uint32_t)((wave * G::DA + q) * 1024), da.off[q] + kg * da.kstep);
-        else dma16(live ? rb : rb_none, slot + D_OPB + (uint32_t)((wave * G::DB + q - G::DA) * 1024), db.off[q - G::DA] + kg * db.kstep);
+        const uint32_t end = KT && kg == k_last ? ~0u : 0u;
+        if (q < G::DA) dma16(live ? ra : ra_none, slot + (uint32_t)((wave * G::DA + q) * 1024),
+                             da.off[q] + kg * da.kstep + (KT && AK ? da.tail[q] & end : 0u));
+        else dma16(live ? rb : rb_none, slot + D_OPB + (uint32_t)((wave * G::DB + q - G::DA) * 1024),
+                   db.off[q - G::DA] + kg * db.kstep + (KT && BK ? db.tail[q - G::DA] & end : 0u));
     };
 
     f32x4 acc[D_FM][D_FN];
@@ -318,9 +327,9 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
     };
 
     if (p.split > 1) {
-        // float32 partials part[z][batch][M][N]
-        float* part = p.part + ((int64_t)blockIdx.z * p.batch + b) * p.M * p.N;
-        if (p.N % 4 == 0 && (reinterpret_cast<uintptr_t>(p.part) & 15) == 0) {
+        // float32 partials part[z][batch][M][np]
+        float* part = p.part + ((int64_t)blockIdx.z * p.batch + b) * p.M * p.np;
+        if (p.np % 4 == 0 && (reinterpret_cast<uintptr_t>(p.part) & 15) == 0) {
             // through the LDS tile: 16-byte row chunks a thread (a lane's
             // accumulators hold four rows of one column; stored directly they
             // are 4-byte stores, which took 2.1 us a workgroup at 128x128)
@@ -337,7 +346,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                     const int rl = q / (D_BN / 4), cc = (q % (D_BN / 4)) * 4;
                     const int row = m0 + pass * 64 + rl, col = n0 + cc;
                     if (row < p.M && col < p.N)
-                        *reinterpret_cast<f32x4*>(part + (int64_t)row * p.N + col) = *reinterpret_cast<const f32x4*>(et + rl * E_LD + cc);
+                        *reinterpret_cast<f32x4*>(part + (int64_t)row * p.np + col) = *reinterpret_cast<const f32x4*>(et + rl * E_LD + cc);
                 }
                 __syncthreads();
             }
@@ -353,7 +362,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int row = m0 + wm * D_WTM + i * 16 + (lane / 16) * 4 + r;
-                    if (row < p.M) part[(int64_t)row * p.N + col] = acc[i][j][r];
+                    if (row < p.M) part[(int64_t)row * p.np + col] = acc[i][j][r];
                 }
             }
         return;
@@ -421,7 +430,8 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
     T* Cb = reinterpret_cast<T*>(p.c) + c_boff(p, b);
     const T* Bb = p.has_bias ? reinterpret_cast<const T*>(p.bias) + bias_boff(p, b) : nullptr;
     auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
-    const bool vec_c = p.sc[2] == 1 && p.sc[1] % 8 == 0 && al16(Cb);
+    // contiguous output rows: 16-byte stores, of any alignment
+    const bool vec_c = p.sc[2] == 1;
     const bool vec_b = p.has_bias && p.sbias[2] == 1 && p.sbias[1] % 8 == 0 && al16(Bb);
     const bool plain = !p.has_bias && p.act == TVK_ACT_NONE;
     // thread tid finishes chunk q = tid + j * D_NT (j < 4) of each 64-row pass:
@@ -431,7 +441,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
     static_assert(CPT * D_NT == 64 * (D_BN / 8), "whole chunks per thread");
     static_assert(64 * (D_BN + 4) * 4 <= D_NS * D_STB, "epilogue tile fits the ring");
     if (plain && vec_c) {
-        // No bias, no activation, 16-byte output rows (most products): each
+        // No bias, no activation, contiguous output rows (most products): each
         // element is its sum times alpha, rounded once, as in the general loop
         // below, with no per-element branches and no bias registers live.
         // (The general loop spends about 500 instructions a chunk on its
@@ -458,7 +468,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                 }
                 T* cp = Cb + (int64_t)row * p.sc[1] + col;
                 if (col + 8 <= p.N) {
-                    st_nt(reinterpret_cast<u32x4*>(cp), u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
+                    st_nt(reinterpret_cast<u32x4u*>(cp), u32x4u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
                                                           (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)});
                 } else {
                     for (int e = 0; e < 8 && col + e < p.N; ++e) cp[e] = __builtin_bit_cast(T, h[e]);
@@ -482,7 +492,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
             }
     }
     if (vec_c && p.act != TVK_ACT_GELU && (!p.has_bias || vec_b)) {
-        // 16-byte output rows, no GELU, and a bias with 16-byte rows or ReLU:
+        // contiguous output rows, no GELU, and a bias with 16-byte rows or ReLU:
         // the epilogue of the general loop below (sum times alpha, plus bias
         // times beta, ReLU, one rounding) with selects in place of its
         // per-element branches
@@ -529,7 +539,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                 }
                 T* cp = Cb + (int64_t)row * p.sc[1] + col;
                 if (full) {
-                    st_nt(reinterpret_cast<u32x4*>(cp), u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
+                    st_nt(reinterpret_cast<u32x4u*>(cp), u32x4u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
                                                           (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)});
                 } else {
                     for (int e = 0; e < 8 && col + e < p.N; ++e) cp[e] = __builtin_bit_cast(T, h[e]);
@@ -582,7 +592,7 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
             }
             T* cp = Cb + (int64_t)row * p.sc[1] + (int64_t)col * p.sc[2];
             if (vec_c && full) {
-                st_nt(reinterpret_cast<u32x4*>(cp), u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
+                st_nt(reinterpret_cast<u32x4u*>(cp), u32x4u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
                                                       (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)});
             } else {
                 for (int e = 0; e < 8 && col + e < p.N; ++e) cp[(int64_t)e * p.sc[2]] = __builtin_bit_cast(T, h[e]);
@@ -601,13 +611,19 @@ void launch_dma_tile(GemmArgs& p, bool a_kmajor, bool b_kmajor, hipStream_t s) {
     p.tiles_n = (p.N + BN - 1) / BN;
     const dim3 grid(p.tiles_m * p.tiles_n, p.batch, p.split > 1 ? p.split : 1), block(DCfg<BM, BN>::NT);
     if constexpr (DCfg<BM, BN>::BIG) {
-        if (p.has_bias && p.split <= 1) {
+        if (p.has_bias && p.split <= 1 && !p.kmask) {
             if (a_kmajor && b_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, true, true, BM, BN, NS, true>), grid, block, 0, s, p);
             else if (a_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, true, false, BM, BN, NS, true>), grid, block, 0, s, p);
             else if (b_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, false, true, BM, BN, NS, true>), grid, block, 0, s, p);
             else hipLaunchKernelGGL((gemm16_dma_kernel<DT, false, false, BM, BN, NS, true>), grid, block, 0, s, p);
             return;
         }
+    }
+    if constexpr (NS == 4 && !(BM == 256 && BN == 128)) if (p.kmask) {
+        if (a_kmajor && b_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, true, true, BM, BN, NS, false, true>), grid, block, 0, s, p);
+        else if (a_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, true, false, BM, BN, NS, false, true>), grid, block, 0, s, p);
+        else hipLaunchKernelGGL((gemm16_dma_kernel<DT, false, true, BM, BN, NS, false, true>), grid, block, 0, s, p);
+        return;
     }
     if (a_kmajor && b_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, true, true, BM, BN, NS>), grid, block, 0, s, p);
     else if (a_kmajor) hipLaunchKernelGGL((gemm16_dma_kernel<DT, true, false, BM, BN, NS>), grid, block, 0, s, p);

@@ -4,9 +4,9 @@
 
 namespace tvk {
 
-bool dma_applies(const GemmArgs& p, bool a_kmajor, bool b_kmajor) {
+bool dma_applies(const GemmArgs& p, bool a_kmajor, bool b_kmajor, bool edges) {
     // K off the 32 grid: the last k step runs whole, so its loads past K must read zeros
-    if (p.K < D_BK || (p.K % D_BK != 0 && !p.kzero)) return false;
+    if (p.K < D_BK || (p.K % D_BK != 0 && (!p.kzero || (p.kmask && !edges)))) return false;
     auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
     if (!al16(p.a) || !al16(p.b)) return false;
     if (p.batch > 1 && (p.sa[0] % 8 != 0 || p.sb[0] % 8 != 0)) return false;
@@ -20,9 +20,9 @@ bool dma_applies(const GemmArgs& p, bool a_kmajor, bool b_kmajor) {
     // an m/n-contiguous operand whose last chunk straddled M or N would lose
     // the valid part of that chunk on the last k-row: the range check ends
     // the buffer at the last element, and extending it would read memory the
-    // tensor may not own
-    if (!a_kmajor && p.M % 8 != 0) return false;
-    if (!b_kmajor && p.N % 8 != 0) return false;
+    // tensor may not own (a repacked operand's range covers its padding)
+    if (!a_kmajor && p.M % 8 != 0 && !(edges && p.a_ext)) return false;
+    if (!b_kmajor && p.N % 8 != 0 && !(edges && p.b_ext)) return false;
     return true;
 }
 

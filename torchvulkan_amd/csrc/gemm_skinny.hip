@@ -506,6 +506,7 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
     if (kring_applies(p, b_kmajor, vec)) {
         GemmArgs q = p;
         const KringShape ks = kring_shape(p);
+        q.np = q.N;
         q.split = ks.split;
         q.k_chunk = ks.chunk;
         Scratch scratch;
@@ -529,6 +530,7 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
     }
     if (ring_applies(p, b_kmajor, vec)) {
         GemmArgs q = p;
+        q.np = q.N;
         q.split = ring_splits(p);
         q.k_chunk = p.K / q.split;
         Scratch scratch;
