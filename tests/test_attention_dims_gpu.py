@@ -77,3 +77,27 @@ def test_masks_of_the_lowest_value(gpu, dtype, dim):
     if dtype == torch.bfloat16:
         bias[:, :, 5] = low   # in float16 the scores do not vanish beside 65504, and the row is an ordinary one
     check(q, k, v, bias=bias, what=f"{dtype} D {dim}")
+
+
+# the 128-query kernel with K and V loaded straight into LDS: the smallest grids that take it, lengths around its
+# query blocks and key tiles, both LDS row widths, sliced keys whose further rows and columns are NaN
+@pytest.mark.parametrize("dim,batch,heads", [(128, 16, 32), (104, 16, 32), (80, 16, 32), (64, 32, 32), (40, 32, 32)])
+@pytest.mark.parametrize("lens,causal", [((127, 127), True), ((128, 64), False), ((100, 65), False), ((70, 200), True)])
+def test_wide_kernel(gpu, dim, batch, heads, lens, causal):
+    from torchvulkan_amd import _abi
+
+    dtype = torch.float16 if dim % 16 else torch.bfloat16
+    n, s = lens
+    q = rand((batch, n, heads, dim), dtype, 1).to(DEV).transpose(1, 2)
+    base = torch.full((batch, s + 9, 2, dim + 8), float("nan"), dtype=dtype)
+    base[:, :s, :, :dim] = rand((batch, s, 2, dim), dtype, 2)
+    kv = base.to(DEV)[:, :s, :, :dim].transpose(1, 2)
+    out, lse = _abi.attention_fwd(q, kv, kv, None, causal, -0.1)
+    torch.cuda.synchronize()
+    for b, h in ((0, 0), (3, heads // 2), (batch - 1, heads - 1)):
+        hk = h // (heads // 2)
+        ro, rl = orc.attention(f64(q[b:b + 1, h:h + 1]), f64(kv[b:b + 1, hk:hk + 1]), f64(kv[b:b + 1, hk:hk + 1]), None,
+                               causal, -0.1)
+        assert_close(f64(out[b:b + 1, h:h + 1]), ro, dtype, f"b {b} h {h}")
+        assert (abs(f64(lse[b:b + 1, h:h + 1]) - rl) <= 1e-3 * (abs(rl) + 1)).all()
+    assert not out.isnan().any()

@@ -40,6 +40,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace tvk {
 
@@ -451,6 +452,231 @@ void attn_fwd_kernel(AttnArgs p) {
     }
 }
 
+// ---------------------------------------------------------------------------
+// The forward on long grids: 4 waves x 32 queries, K and V by loads straight
+// into LDS.
+// ---------------------------------------------------------------------------
+// The same orientation and softmax as attn_fwd_kernel; what differs is what
+// bounds that kernel on long sequences:
+//   - LDS reads. With 16 queries a wave every K and V fragment feeds one
+//     product: at head_dim 128 a 64-key tile costs a wave 256 cycles of the
+//     CU's one LDS pipe against 512 of its own matrix pipe, so four waves are
+//     bound by LDS. Two 16-query columns a wave halve that.
+//   - Registers. Two columns at head_dim 128 with two tiles staged in
+//     registers need over 256; loads straight into LDS need none for staging
+//     (204 VGPRs, two waves a SIMD, two workgroups a CU of 64 KB each). Rows
+//     stay 256 (head dims above 64) or 128 bytes with their 16-byte chunks
+//     XOR-swizzled, which the loads allow where row padding would not fit
+//     their contiguous 1 KB blocks.
+// bfloat16 2 x 32/8 heads x 3001 x 128 causal: 242 -> 178 us (0.83 PFLOP/s);
+// 8 x 32/8 x 256 x 128: 22.2 -> 15.9; 8 x 16 x 577 x 80 full: 48.0 -> 37.4; 8 x
+// 16 x 4096 x 64: 417 -> 366. What is left is waiting: matrix, vector and LDS
+// pipes each need about a third of the time (raising a wave's priority around
+// its products moved nothing).
+typedef int i32x4v __attribute__((ext_vector_type(4)));
+
+// Buffer resource of the largest 32-bit range at p; offsets at or past kOOB read zeros.
+__device__ inline i32x4v attn_rsrc(const char* p) {
+    const uint64_t a = (uint64_t)p;
+    return i32x4v{(int)(uint32_t)a, (int)((a >> 32) & 0xffff), 0x7fffffff, 0x00020000};
+}
+// 16 bytes per lane into LDS at lds_addr + 16 * lane. From asm, so that the
+// compiler does not hold every later LDS read behind it; the waits are explicit.
+__device__ inline void attn_dma16(i32x4v r, uint32_t lds_addr, uint32_t voff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                 :: "s"(lds_addr), "v"(voff), "s"(r) : "memory");
+}
+
+template <int DT, int D, bool CAUSAL, bool PART>
+__global__ __launch_bounds__(64 * AT_WAVES, 2) void attn_fwd_wide_kernel(AttnArgs p) {
+    constexpr int QPW = 2, BMQ = 16 * QPW * AT_WAVES;
+    constexpr int DS = D / 32, DT16 = D / 16;
+    constexpr int RB = D > 64 ? 256 : 128;            // bytes of an LDS row
+    constexpr int CPR = RB / 16;                      // its 16-byte chunks
+    constexpr int TB = AT_BN * RB;                    // bytes of a K or V tile
+    constexpr int LPW = TB / 1024 / AT_WAVES;         // loads per wave and tile
+    __shared__ __attribute__((aligned(1024))) char lds[2][2][TB];   // [buffer][K, V]
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TVK_LDS char*)&lds[0][0][0]);
+
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int g = lane / 16, c16 = lane % 16;
+    int qb, bh;
+    attn_block<CAUSAL>(p, qb, bh);
+    const int b = bh / p.Hq, h = bh % p.Hq;
+    const int hk = h / p.group;
+    const int q0 = qb * BMQ + wave * 16 * QPW;   // this wave's first query
+
+    // LDS slot of chunk c of row r: K rows are read 16 at one chunk, V rows
+    // (transposed) 8 at one chunk pair; either way a served group of lanes
+    // meets all 64 banks once
+    auto kswz = [](int r) { return CPR == 16 ? r & 15 : (r >> 1) & 7; };
+    auto vswz = [](int r) { return CPR == 16 ? (r & 7) * 2 : ((r >> 1) & 3) * 2; };
+
+    const char* Kh = reinterpret_cast<const char*>(p.k + (int64_t)b * p.sk[0] + (int64_t)hk * p.sk[1]);
+    const char* Vh = reinterpret_cast<const char*>(p.v + (int64_t)b * p.sv[0] + (int64_t)hk * p.sv[1]);
+    const int64_t kstep = (int64_t)AT_BN * p.sk[2] * 2, vstep = (int64_t)AT_BN * p.sv[2] * 2;
+    uint32_t koff[LPW], voff[LPW];
+    int row[LPW];
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) {
+        row[i] = (wave * LPW + i) * (64 / CPR) + lane / CPR;
+        const int kc = (lane % CPR) ^ kswz(row[i]), vc = (lane % CPR) ^ vswz(row[i]);
+        // chunks past the head dim read zeros
+        koff[i] = kc * 8 < (PART ? p.hd : D) ? (uint32_t)((row[i] * (int)p.sk[2] + kc * 8) * 2) : kOOB;
+        voff[i] = vc * 8 < (PART ? p.hd : D) ? (uint32_t)((row[i] * (int)p.sv[2] + vc * 8) * 2) : kOOB;
+    }
+    auto issue = [&](int j) {
+        const i32x4v rk = attn_rsrc(Kh + j * kstep), rv = attn_rsrc(Vh + j * vstep);
+        const uint32_t at = lds0 + (uint32_t)((j & 1) * 2 * TB + wave * LPW * 1024);
+        const bool whole = j * AT_BN + AT_BN <= p.S;   // rows past the last key are zeros: P is 0 there and V must be finite
+#pragma unroll
+        for (int i = 0; i < LPW; ++i) attn_dma16(rk, at + i * 1024, whole || j * AT_BN + row[i] < p.S ? koff[i] : kOOB);
+#pragma unroll
+        for (int i = 0; i < LPW; ++i) attn_dma16(rv, at + TB + i * 1024, whole || j * AT_BN + row[i] < p.S ? voff[i] : kOOB);
+    };
+
+    int ntiles = (p.S + AT_BN - 1) / AT_BN;
+    if (CAUSAL) {
+        const int last_q = min(p.L, qb * BMQ + BMQ) - 1;   // keys beyond it are masked for the block
+        ntiles = min(ntiles, last_q / AT_BN + 1);
+    }
+    if (ntiles > 0) issue(0);
+
+    // Q^T as the B operand: lane holds query q0+16qt+c16, d = 32ds + 8g .. +7
+    const uint16_t* Q = p.q + (int64_t)b * p.sq[0] + (int64_t)h * p.sq[1];
+    u32x4 qf[QPW][DS];
+#pragma unroll
+    for (int qt = 0; qt < QPW; ++qt) {
+        const int qi = q0 + 16 * qt + c16;
+#pragma unroll
+        for (int ds = 0; ds < DS; ++ds) {
+            const bool in = qi < p.L && (!PART || 32 * ds + 8 * g < p.hd);
+            u32x4 x = in ? *reinterpret_cast<const u32x4*>(Q + (int64_t)qi * p.sq[2] + 32 * ds + 8 * g) : u32x4{0, 0, 0, 0};
+            x ^= p.qflip;
+            qf[qt][ds] = x;
+        }
+    }
+    f32x4 oacc[DT16][QPW];
+#pragma unroll
+    for (int i = 0; i < DT16; ++i)
+#pragma unroll
+        for (int qt = 0; qt < QPW; ++qt) oacc[i][qt] = f32x4{0, 0, 0, 0};
+    float m_run[QPW], l_run[QPW];   // m in log2 units; l a per-lane partial sum
+#pragma unroll
+    for (int qt = 0; qt < QPW; ++qt) {
+        m_run[qt] = -INFINITY;
+        l_run[qt] = 0.0f;
+    }
+    // per-lane LDS offsets: K row c16 of a 16-row block at chunk 4ds + g; V row
+    // 4g + c16/4 of a 16-row block, four columns from 4 (c16 % 4) of tile i
+    uint32_t kat[DS], vat[DT16];
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) kat[ds] = lds0 + c16 * RB + (((4 * ds + g) ^ kswz(c16)) * 16);
+    const int vr = 4 * g + c16 / 4;
+#pragma unroll
+    for (int i = 0; i < DT16; ++i) vat[i] = lds0 + TB + vr * RB + (((2 * i + (c16 % 4) / 2) ^ vswz(vr)) * 16) + (c16 % 2) * 8;
+
+    auto compute_tile = [&](int j, auto buf_c) {
+        constexpr uint32_t buf = decltype(buf_c)::value * 2 * TB;   // an offset of the LDS reads
+        const int k0 = j * AT_BN;
+        // a causal wave whose queries all precede the tile has nothing to add
+        if (CAUSAL && k0 > q0 + 16 * QPW - 1) return;
+        // ---- S^T = K Q^T over 4 key blocks x QPW query columns
+        f32x4 sacc[4][QPW];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+#pragma unroll
+            for (int qt = 0; qt < QPW; ++qt) sacc[kt][qt] = f32x4{0, 0, 0, 0};
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) {
+                const u32x4 kf = *(const TVK_LDS u32x4*)(uintptr_t)(kat[ds] + buf + kt * 16 * RB);
+#pragma unroll
+                for (int qt = 0; qt < QPW; ++qt) sacc[kt][qt] = mfma16<DT>(kf, qf[qt][ds], sacc[kt][qt]);
+            }
+        }
+        // ---- online softmax per query column
+        float alpha[QPW];
+        if (k0 + AT_BN <= p.S && !(CAUSAL && k0 + AT_BN - 1 > q0))
+            softmax_tile<DT, true, false, CAUSAL, QPW>(p, sacc, m_run, l_run, alpha, k0, q0, b, h, g, c16);
+        else
+            softmax_tile<DT, false, false, CAUSAL, QPW>(p, sacc, m_run, l_run, alpha, k0, q0, b, h, g, c16);
+        bool rescale = false;
+#pragma unroll
+        for (int qt = 0; qt < QPW; ++qt) rescale = rescale || alpha[qt] != 1.0f;
+        if (__any(rescale)) {
+#pragma unroll
+            for (int i = 0; i < DT16; ++i)
+#pragma unroll
+                for (int qt = 0; qt < QPW; ++qt)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) oacc[i][qt][r] *= alpha[qt];
+        }
+        // ---- O^T += V^T P^T: two 32-key products, k-slots in the S^T lane order
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            u32x4 pf[QPW];
+#pragma unroll
+            for (int qt = 0; qt < QPW; ++qt) {
+                const f32x4 a = sacc[2 * kk][qt], c = sacc[2 * kk + 1][qt];
+                pf[qt] = u32x4{pack2<DT>(a[0], a[1]), pack2<DT>(a[2], a[3]), pack2<DT>(c[0], c[1]), pack2<DT>(c[2], c[3])};
+            }
+#pragma unroll
+            for (int i = 0; i < DT16; ++i) {
+                u32x4 vf;
+#pragma unroll
+                for (int rr = 0; rr < 2; ++rr) {
+                    TVK_LDS s16x4* ptr = (TVK_LDS s16x4*)(uintptr_t)(vat[i] + buf + (2 * kk + rr) * 16 * RB);
+                    const u32x2 w = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(ptr));
+                    vf[2 * rr] = w.x;
+                    vf[2 * rr + 1] = w.y;
+                }
+#pragma unroll
+                for (int qt = 0; qt < QPW; ++qt) oacc[i][qt] = mfma16<DT>(vf, pf[qt], oacc[i][qt]);
+            }
+        }
+    };
+
+    auto step = [&](int j, auto buf_c) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's loads of tile j have landed
+        __syncthreads();   // every wave's have, and every wave has left tile j - 1's buffer
+        if (j + 1 < ntiles) issue(j + 1);
+        compute_tile(j, buf_c);
+    };
+    for (int j = 0; j < ntiles; j += 2) {
+        step(j, std::integral_constant<uint32_t, 0>{});
+        if (j + 1 < ntiles) step(j + 1, std::integral_constant<uint32_t, 1>{});
+    }
+
+    // ---- O = O^T / l; lse = m ln2 + log l (+inf for a row that attended to nothing)
+    float l_tot[QPW];
+#pragma unroll
+    for (int qt = 0; qt < QPW; ++qt) l_tot[qt] = lanes4_sum(l_run[qt]);   // every lane, before any divergence
+    uint16_t* O = p.out + (int64_t)b * p.so[0] + (int64_t)h * p.so[1];
+#pragma unroll
+    for (int qt = 0; qt < QPW; ++qt) {
+        const int qi = q0 + 16 * qt + c16;
+        if (qi >= p.L) continue;
+        const float inv = l_tot[qt] > 0.0f ? 1.0f / l_tot[qt] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < DT16; ++i) {
+            const int dv = 16 * i + 4 * g;   // four consecutive dv of column qi
+            if (PART && dv >= p.hd) continue;
+            const f32x4 o = oacc[i][qt];
+            uint16_t* op = O + (int64_t)qi * p.so[2] + (int64_t)dv * p.so[3];
+            if (p.out_vec) {
+                *reinterpret_cast<u32x2*>(op) = u32x2{pack2<DT>(o[0] * inv, o[1] * inv), pack2<DT>(o[2] * inv, o[3] * inv)};
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    op[(int64_t)r * p.so[3]] = __builtin_bit_cast(uint16_t, elem<DT>::from_f32(o[r] * inv));
+            }
+        }
+        if (g == 0)
+            p.lse[(int64_t)b * p.sl[0] + (int64_t)h * p.sl[1] + (int64_t)qi * p.sl[2]] =
+                l_tot[qt] > 0.0f ? m_run[qt] * AT_LN2 + logf(l_tot[qt]) : INFINITY;
+    }
+}
+
 template <int DT, int D, int QPW, bool PART>
 void launch_attn_q(AttnArgs a, bool causal, bool bias, int64_t bh, int64_t L, hipStream_t s) {
     constexpr int BMQ = 16 * QPW * AT_WAVES;
@@ -466,12 +692,27 @@ void launch_attn_q(AttnArgs a, bool causal, bool bias, int64_t bh, int64_t L, hi
     }
 }
 
-// Query columns per wave: at head_dim 64, two (128 queries per workgroup) when
-// that still gives the device plenty of workgroups, else one (64 per
-// workgroup). At head_dim 128 two columns need over 256 VGPRs (one wave per
-// SIMD), so it is always one; so do the PART kernels.
+// Two query columns a wave (the wide kernel) where its 128-query workgroups
+// still fill the device: from two a CU (head_dim 128, 8 heads x 4608: 288 of
+// them, 94 us on the 64-query kernel, 138 wide; 512 of them, 22.2 against 17.0),
+// at head_dim 64, where less LDS lets more of the 64-query workgroups share a
+// CU, from four (512 of 32 x 8 x 256: 10.76 against 10.86; 1024 of 16 x 16 x
+// 512: 35.2 against 31.3). With a bias the 64-query kernel, at head_dim 64 on
+// large grids in its two-column form.
 template <int DT, int D, bool PART>
 void launch_attn(const AttnArgs& a, bool causal, bool bias, int64_t batch, int64_t heads, int64_t L, hipStream_t s) {
+    if constexpr (D >= 64) {
+        const bool rows_ok = (AT_BN * a.sk[2] + 128) * 2 < (int64_t)0x7fffffff && (AT_BN * a.sv[2] + 128) * 2 < (int64_t)0x7fffffff;
+        if (!bias && rows_ok && batch * heads * ((L + 127) / 128) >= (D == 64 ? 1024 : 512)) {
+            AttnArgs w = a;
+            w.nqb = (int)((L + 127) / 128);
+            w.BH = (int)(batch * heads);
+            const dim3 grid((unsigned)(w.nqb * w.BH)), block(64 * AT_WAVES);
+            if (causal) hipLaunchKernelGGL((attn_fwd_wide_kernel<DT, D, true, PART>), grid, block, 0, s, w);
+            else hipLaunchKernelGGL((attn_fwd_wide_kernel<DT, D, false, PART>), grid, block, 0, s, w);
+            return;
+        }
+    }
     if constexpr (D == 64 && !PART) {
         if (batch * heads * ((L + 127) / 128) >= 2048) {
             launch_attn_q<DT, D, 2, PART>(a, causal, bias, batch * heads, L, s);
