@@ -67,6 +67,7 @@ FILE_FLAGS = {
     "attention_part.hip": VGPR_FORM,
     "calibrate.hip": VGPR_FORM,
     "gemm_dma128.hip": VGPR_FORM,
+    "gemm_seq_ring.hip": VGPR_FORM,
     "gemm_skinny.hip": VGPR_FORM,
     "conv.hip": VGPR_FORM,
     "conv_nhwc.hip": VGPR_FORM,

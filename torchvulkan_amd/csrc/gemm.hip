@@ -504,8 +504,8 @@ __global__ __launch_bounds__(256) void gemm_seq_mfma_kernel(GemmArgs p) {
         }
 }
 
-// The same order on 64x64 tiles for products with few tiles (1024^2 float32:
-// 256 tiles against 128 of 64x128): each of the four waves owns 16 rows x 64
+// The same order on 64x64 tiles for 16-bit products with few tiles (float32:
+// gemm_seq_ring.hip): each of the four waves owns 16 rows x 64
 // columns and issues v_mfma_f32_16x16x1_4b_f32 with its row's A value in all
 // four blocks, so one instruction is a 16x64 rank-1 update (block q: columns
 // 16q .. 16q+15), at the matrix core's float32 rate like the 32x32x1 form.
@@ -1232,7 +1232,8 @@ tvk_status run(const tvk_gemm_desc& d, const Plan& pl, hipStream_t s, char* fixe
             q.tiles_m = (int)((d.M + 63) / 64);
             q.tiles_n = (int)((d.N + 63) / 64);
             dim3 grid(q.tiles_m * q.tiles_n, nb);
-            launch_seq16<DT>(pl, q, grid, s);
+            if constexpr (DT == TVK_F32) launch_seq_ring(q, pl.ak, pl.bk, pl.vec, s);
+            else launch_seq16<DT>(pl, q, grid, s);
             break;
         }
         case Kern::SEQ128:

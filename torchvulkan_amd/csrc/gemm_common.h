@@ -443,6 +443,9 @@ __device__ inline u32x4 load_chunk(__amdgpu_buffer_rsrc_t r, bool row_ok, int64_
 // edges: also the products whose last k step needs masks (kmask) or whose
 // m/n-contiguous rows end inside a 16-byte chunk of a repacked operand.
 bool dma_applies(const GemmArgs& p, bool a_kmajor, bool b_kmajor, bool edges = false);
+// float32 in sequential order on 64x64 tiles (tiles_m, tiles_n set; gemm_seq_ring.hip). vec: 16-byte chunks of both
+// operands' contiguous dimension are whole and aligned.
+void launch_seq_ring(const GemmArgs& p, bool a_kmajor, bool b_kmajor, bool vec, hipStream_t s);
 // tile: 256 (256x256), 128 (128x128), DMA_TILE_128X256 or DMA_TILE_256X128
 constexpr int DMA_TILE_128X256 = 1, DMA_TILE_256X128 = 2;
 hipError_t launch_dma(int dtype, GemmArgs& p, bool a_kmajor, bool b_kmajor, int tile, hipStream_t s, int stages = 4);
