@@ -73,3 +73,22 @@ def test_every_family_of_an_odd_plane(gpu):
         torch.cuda.synchronize()
         assert torch.equal(dw.cpu().double(), want), name
     _abi.tune_reset()
+
+
+def test_captured_grad_weight(gpu):
+    # a captured call allocates nothing: on a stream whose workspace pool is empty, a short reduction is captured,
+    # replayed between eager calls, and gives the eager result every time
+    x, dy = (ints(s, i, -1, 1).half().to(DEV) for i, s in enumerate([(2, 32, 14, 14), (2, 24, 14, 14)]))
+    want = torch.nn.grad.conv2d_weight(x.cpu().double(), (24, 32, 3, 3), dy.cpu().double(), padding=1)
+    dw = torch.empty((24, 32, 3, 3), dtype=torch.float16, device=DEV)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        d = _abi.conv_problem(x, dw, dy, padding=1)
+        _abi.conv_run(d, _abi.TVK_CONV_WGRAD)
+    for _ in range(3):
+        dw.zero_()
+        graph.replay()
+        eager = _abi.conv2d_wgrad(x, dy, (24, 32, 3, 3), padding=1)
+        torch.cuda.synchronize()
+        assert torch.equal(dw.cpu().double(), want) and torch.equal(eager.cpu().double(), want)

@@ -737,7 +737,16 @@ tvk_status run_family(const tvk_conv_desc& d, ConvFamily f, const char* who) {
     if (p.N != 0 && p.M != 0 && p.K != 0) {
         if (f == ConvFamily::SMALL) return conv_small_run(d, MODE, who);
         if (f == ConvFamily::HALO) return conv_halo_run(d, MODE, who);
-        if (f == ConvFamily::RING) return conv_ring_run(d, MODE, who);
+        if (f == ConvFamily::RING) {
+            if (!conv_ring_dy_last(d, MODE)) return conv_ring_run(d, MODE, who);
+            // The generic kernel takes these planes too and needs less workspace, or none on short reductions: it runs
+            // where the copies' workspace is not to be had (a captured call must not allocate it).
+            if (scratch_usable(resolve_stream(d.stream))) {
+                const tvk_status st = conv_ring_run(d, MODE, who);
+                if (st != TVK_ERR_OOM) return st;
+                clear_error();
+            }
+        }
     }
     return run_generic<2, MODE>(p, d.dtype, (d.flags & TVK_GEMM_EXACT) != 0, p.out, resolve_stream(d.stream), who);
 }

@@ -676,6 +676,18 @@ void border_for(int lo, int step, int count, int tap_lo, int tap_hi, int size, i
     after = std::max(after, lo + (count - 1) * step + tap_hi - (size - 1));
 }
 
+// The border of a grad weight's channels-last x, and that copy's bytes (16-bit elements).
+Border wgrad_border(const tvk_conv_desc& d) {
+    Border bd;
+    border_for(-(int)d.padding[0], (int)d.stride[0], (int)d.h_out, 0, (int)((d.kh - 1) * d.dilation[0]), (int)d.h, bd.pt, bd.pb);
+    border_for(-(int)d.padding[1], (int)d.stride[1], (int)d.w_out, 0, (int)((d.kw - 1) * d.dilation[1]), (int)d.w, bd.pl, bd.pr);
+    return bd;
+}
+
+int64_t wgrad_bordered_bytes(const tvk_conv_desc& d, const Border& bd) {
+    return d.n * d.c_in * (d.h + bd.pt + bd.pb) * (d.w + bd.pl + bd.pr) * 2;
+}
+
 // ---------------------------------------------------------------------------
 // Stride-1 3x3 "same" convolution (padding 1) straight from NCHW: forward
 // (source x) and grad input (source dy, taps mirrored). A workgroup computes
@@ -2087,6 +2099,8 @@ __global__ __launch_bounds__(256) void conv1x1_dgrad_kernel(PointDgArgs p) {
 }  // namespace
 
 // mode: 0 forward, 1 grad input, 2 grad weight
+bool conv_ring_dy_last(const tvk_conv_desc& d, int mode) { return mode == 2 && (d.h_out * d.w_out) % 32 != 0; }
+
 bool conv_ring_applies(const tvk_conv_desc& d, int mode) {
     if (d.dtype != TVK_F16 && d.dtype != TVK_BF16) return false;
     if ((d.flags & TVK_GEMM_EXACT) || d.groups != 1) return false;
@@ -2101,8 +2115,10 @@ bool conv_ring_applies(const tvk_conv_desc& d, int mode) {
     auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
     if (!al16(d.x) || !al16(d.weight) || !al16(d.y)) return false;
     if (mode == 1 && (d.stride[0] > 4 || d.stride[1] > 4)) return false;
-    // planes of other than whole 32-pixel stages read dy channels-last, in 8-channel chunks
-    if (mode == 2 && (d.h_out * d.w_out) % 32 != 0 && d.c_out % 8 != 0) return false;
+    // planes of other than whole 32-pixel stages read dy channels-last, in 8-channel chunks; the generic kernel takes
+    // the ones whose bordered copy would pass 2 GiB
+    if (conv_ring_dy_last(d, mode) && (d.c_out % 8 != 0 || wgrad_bordered_bytes(d, wgrad_border(d)) >= (int64_t(1) << 31)))
+        return false;
     // 32-bit element offsets inside the kernels
     const int64_t big = std::max({d.n * d.c_in * d.h * d.w, d.n * d.c_out * d.h_out * d.w_out, d.c_out * d.c_in * d.kh * d.kw});
     return big < (int64_t(1) << 30);
@@ -2245,12 +2261,10 @@ tvk_status conv_ring_run(const tvk_conv_desc& d, int mode, const char* who) {
         // channels-last with x in one launch (the element-gathering kernel of conv.hip took such planes before:
         // bfloat16 32 x 128 x 28 x 28 to 128 channels, 3x3: 132 us there; 36 here, 22 of them the products); K =
         // output pixels split into partials
-        const bool dy_last = (Ho * Wo) % 32 != 0;
-        Border bd;
-        border_for(-ph, sh, Ho, 0, (kh - 1) * dh, H, bd.pt, bd.pb);
-        border_for(-pw, sw, Wo, 0, (kw - 1) * dw, W, bd.pl, bd.pr);
+        const bool dy_last = conv_ring_dy_last(d, mode);
+        const Border bd = wgrad_border(d);
         const int Hs = H + bd.pt + bd.pb, Ws = W + bd.pl + bd.pr;
-        if ((size_t)n * cin * Hs * Ws * es >= ((size_t)1 << 31))
+        if (wgrad_bordered_bytes(d, bd) >= (int64_t(1) << 31))
             return fail(TVK_ERR_UNSUPPORTED, std::string(who) + ": the bordered channels-last copy exceeds 2 GiB");
         const size_t act_b = align((size_t)n * cin * Hs * Ws * es), dy_b = dy_last ? align((size_t)n * cout * Ho * Wo * es) : 0;
         p.M = T * cin;

@@ -453,6 +453,8 @@ hipError_t launch_dma(int dtype, GemmArgs& p, bool a_kmajor, bool b_kmajor, int 
 // Channels-last convolution on the LDS ring (conv_nhwc.hip); mode 0 forward,
 // 1 grad input, 2 grad weight.
 bool conv_ring_applies(const tvk_conv_desc& d, int mode);
+// Whether that family copies dy channels-last for the grad weight: planes of other than whole 32-pixel stages.
+bool conv_ring_dy_last(const tvk_conv_desc& d, int mode);
 tvk_status conv_ring_run(const tvk_conv_desc& d, int mode, const char* who);
 // Stride-1 3x3 padding-1 forward / grad input from NCHW through an LDS halo
 // (conv_nhwc.hip); mode 0 or 1.
