@@ -63,7 +63,8 @@ def test_views_batches_and_epilogue(gpu, m):
 
 @pytest.mark.parametrize("m", [16, 64])
 def test_noalloc_and_capture(gpu, m):
-    # without scratch of the pool: the allocation-free entry point sums in a second launch, a captured call runs unsplit
+    # without scratch of the pool: the allocation-free entry point sums in a second launch, a captured call whose
+    # stream has no idle scratch runs unsplit
     dtype = torch.bfloat16
     x, w = operands(m, 512, 8192 if m == 16 else 4096, dtype, 11)
     want = x.double() @ w.double().t()
@@ -82,3 +83,28 @@ def test_noalloc_and_capture(gpu, m):
         _abi.gemm(xd, wd.t(), other)
         torch.cuda.synchronize()
         assert torch.equal(c.cpu().double(), want) and torch.equal(other, c)
+
+
+# K chunks summed in a captured second launch: one strip and several, rows of one, two and four blocks
+@pytest.mark.parametrize("m,n,k", [(17, 64, 2048), (33, 256, 8000), (64, 1000, 4096), (32, 512, 8192)])
+def test_capture_on_a_warm_stream(gpu, m, n, k):
+    # a stream whose pool holds an idle buffer: the captured call splits K like an eager one
+    dtype = torch.bfloat16
+    x, w = operands(m, n, k, dtype, 11)
+    want = x.double() @ w.double().t()
+    xd, wd = x.to(DEV), w.to(DEV)
+    c, e = (torch.full((m, n), 7, dtype=dtype, device=DEV) for _ in range(2))
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        _abi.gemm(xd, wd.t(), e)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        _abi.gemm(xd, wd.t(), c)
+    for _ in range(3):
+        c.fill_(7)
+        graph.replay()
+        _abi.gemm(xd, wd.t(), e)
+        torch.cuda.synchronize()
+        assert torch.equal(c.cpu().double(), want) and torch.equal(e, c)

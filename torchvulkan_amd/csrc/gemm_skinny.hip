@@ -511,10 +511,17 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
         q.k_chunk = ks.chunk;
         Scratch scratch;
         if (q.split > 1 && !part) {
-            // A call without scratch of its own (capture: its pool and counters must not be touched; no memory) runs
-            // unsplit, as this layout always did.
-            const bool can = scratch_usable(s) && (int64_t)q.split * p.batch * p.M * p.N * 4 < (int64_t(1) << 31);
-            q.part = can ? static_cast<float*>(scratch.get((size_t)q.split * p.batch * p.M * p.N * 4, s)) : nullptr;
+            // A call without scratch of its own (capture: its counters must not be touched and it must not allocate; no
+            // memory) runs unsplit, as up to 16 rows always did. Above, the tiled plans split from K = 2048 and lease
+            // scratch also under capture: a captured call does so where the stream's pool holds an idle buffer, and
+            // sums the partials in a second launch (unsplit, few strips leave most CUs idle: bfloat16 33 x 8000 x 256
+            // 29.1 us, 10.9 on split tiles, 9.7 so).
+            const size_t bytes = (size_t)q.split * p.batch * p.M * p.N * 4;
+            const bool fits = bytes < (size_t)1 << 31, usable = scratch_usable(s);
+            const bool idle = !usable && p.M > 16 && p.K >= 2048 && s != hipStreamPerThread;
+            q.part = nullptr;
+            if (fits && usable) q.part = static_cast<float*>(scratch.get(bytes, s));
+            else if (fits && idle) q.part = static_cast<float*>(scratch.get_idle(bytes, s));
             if (q.part) q.tile_count = split_counters(s, (int64_t)ks.strips * p.batch);
             else q.split = 1;
         } else {

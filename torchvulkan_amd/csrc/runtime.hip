@@ -134,11 +134,16 @@ DeviceScratch* device_scratch(int device) {
 
 }  // namespace
 
-void* Scratch::get(size_t bytes, hipStream_t stream) {
+void* Scratch::get(size_t bytes, hipStream_t stream) { return lease(bytes, stream, false); }
+
+void* Scratch::get_idle(size_t bytes, hipStream_t stream) { return lease(bytes, stream, true); }
+
+void* Scratch::lease(size_t bytes, hipStream_t stream, bool idle_only) {
     release();
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
-    auto* buf = device_scratch(dev)->pool.acquire(bytes, stream);
+    auto& pool = device_scratch(dev)->pool;
+    auto* buf = idle_only ? pool.acquire_idle(bytes, stream) : pool.acquire(bytes, stream);
     if (!buf) return nullptr;
     lease_ = buf;
     device_ = dev;

@@ -83,6 +83,19 @@ public:
         return pick;
     }
 
+    // An idle buffer of this stream that is large enough, or nullptr: allocates and frees nothing.
+    Buffer* acquire_idle(size_t bytes, Stream s) {
+        std::lock_guard<std::mutex> lk(mu_);
+        Buffer* pick = nullptr;
+        for (auto& up : bufs_) {
+            Buffer* b = up.get();
+            if (b->held || !(b->stream == s) || b->bytes < bytes) continue;
+            if (!pick || b->bytes < pick->bytes) pick = b;
+        }
+        if (pick) pick->held = true;
+        return pick;
+    }
+
     // Ends a lease; the next lease for the same stream may take the buffer.
     void release(Buffer* buf) {
         if (!buf) return;

@@ -48,9 +48,13 @@ public:
     // on `stream`; NULL when it cannot be allocated. One lease per object: a
     // second call ends the first lease.
     void* get(size_t bytes, hipStream_t stream);
+    // The same from a buffer that the stream's earlier calls have left idle,
+    // NULL without one: allocates nothing, so a captured call may ask.
+    void* get_idle(size_t bytes, hipStream_t stream);
     void release();
 
 private:
+    void* lease(size_t bytes, hipStream_t stream, bool idle_only);
     void* lease_ = nullptr;
     int device_ = -1;
     hipStream_t stream_ = nullptr;
