@@ -102,3 +102,28 @@ def test_two_streams_and_capture(gpu):
         # one split instead of several: the same products merged in another order
         assert_close(f64(out), f64(want[0][0]), dtype, "captured")
         assert torch.allclose(lse, want[0][1], rtol=1e-5, atol=1e-5)
+
+
+# infinities and NaN in V: a column that holds one is that value (or NaN) in every row that attends to it, the other
+# columns are what they are without it. 3, 11 and 8 splits of the keys (the merge works on groups of eight), the value
+# in the first, a middle and the last split; 1 and 40 query rows of a key/value head
+@pytest.mark.parametrize("batch,heads,new,keys", [(2, (16, 16), 1, 700), (1, (8, 1), 1, 1400), (1, (8, 8), 5, 1000),
+                                                  (2, (16, 2), 5, 1400), (1, (40, 1), 1, 1024)])
+@pytest.mark.parametrize("dim", [64, 80, 128])
+def test_non_finite_values(gpu, batch, heads, new, keys, dim):
+    dtype = torch.bfloat16
+    q, k = rand((batch, heads[0], new, dim), dtype, 1) * 0.1, rand((batch, heads[1], keys, dim), dtype, 2) * 0.1
+    v = rand((batch, heads[1], keys, dim), dtype, 3)
+    # (weights are all about 1 / keys: no product of a zero weight)
+    for at, col, value in ((1, 3, float("inf")), (keys // 2, 17, float("-inf")), (keys - 1, 30, float("inf")),
+                           (keys - 2, 31, float("nan"))):
+        v[:, :, at, col] = value
+    out, lse = _abi.attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV))
+    torch.cuda.synchronize()
+    out = f64(out)
+    assert (out[..., 3] == np.inf).all() and (out[..., 17] == -np.inf).all() and (out[..., 30] == np.inf).all()
+    assert np.isnan(out[..., 31]).all()
+    finite = [c for c in range(dim) if c not in (3, 17, 30, 31)]
+    ro, rl = orc.attention(f64(q), f64(k), f64(torch.nan_to_num(v, 0.0, 0.0, 0.0)), None, False)
+    assert_close(out[..., finite], ro[..., finite], dtype, "finite columns")
+    assert np.allclose(f64(lse), rl, rtol=1e-3, atol=1e-3)

@@ -88,7 +88,7 @@ __device__ inline void decode_merge(const DecodeArgs& p, int64_t row, int64_t al
         f32x4 os[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t at = min(s0 + u, p.splits - 1) * all_rows + row;   // past the end: the last split, weight 0
+            const int64_t at = min(s0 + u, p.splits - 1) * all_rows + row;   // past the end: the last split, not added
             w[u] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, decode_ml_at(p, at), 0, kCoherent));
             os[u] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, decode_o_at(p, at, dv), 0, kCoherent));
         }
@@ -102,8 +102,9 @@ __device__ inline void decode_merge(const DecodeArgs& p, int64_t row, int64_t al
         m = mn;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+            if (s0 + u >= p.splits) break;   // (a weight of 0 would make NaN of an infinite sum)
             const float ms = __builtin_bit_cast(float, (uint32_t)w[u][0]), ls = __builtin_bit_cast(float, (uint32_t)w[u][1]);
-            const float f = s0 + u >= p.splits || ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ms - m) * UNIT);
+            const float f = ms == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((ms - m) * UNIT);
             l += ls * f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] += os[u][e] * f;
