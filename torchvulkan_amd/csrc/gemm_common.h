@@ -241,7 +241,7 @@ __device__ __forceinline__ bool finish4_vec(const GemmArgs& p) { return p.sc[2] 
 constexpr int kCoherent = 1 | 16;   // sc0 | sc1: system scope
 
 __device__ inline __amdgpu_buffer_rsrc_t part_rsrc(const GemmArgs& p) {
-    const int64_t bytes = (int64_t)p.split * p.batch * p.M * p.N * 4;
+    const int64_t bytes = (int64_t)p.split * p.batch * p.M * p.np * 4;
     return __builtin_amdgcn_make_buffer_rsrc((void*)p.part, 0, (int)bytes, 0x00020000);
 }
 
@@ -256,7 +256,7 @@ __device__ inline void part_store(__amdgpu_buffer_rsrc_t r, int64_t idx, float v
 // tile's planes in split order with the additions and rounding of
 // gemm_split_reduce4_kernel, so both paths give the same bits. No workgroup
 // waits on another. Tile: rows m0 .. m0 + BM - 1, columns n0 .. n0 + BN - 1
-// of matrix b (N % 4 == 0: 16-byte partial rows). `flag`: one word of LDS
+// of matrix b (np % 4 == 0: 16-byte partial rows). `flag`: one word of LDS
 // that no wave reads, nor loads into, any more.
 template <int DT, int NT, int BM, int BN>
 __device__ void split_fixup(const GemmArgs& p, int b, int m0, int n0, unsigned* cnt, int* flag) {
@@ -271,7 +271,7 @@ __device__ void split_fixup(const GemmArgs& p, int b, int m0, int n0, unsigned* 
     __syncthreads();
     if (!*flag) return;
     const __amdgpu_buffer_rsrc_t r = part_rsrc(p);
-    const int64_t mn = (int64_t)p.M * p.N, total = (int64_t)p.batch * mn;
+    const int64_t mn = (int64_t)p.M * p.np, total = (int64_t)p.batch * mn;
     auto ld = [&](int64_t idx) {
         return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)(idx * 4), 0, kCoherent));
     };
@@ -280,7 +280,7 @@ __device__ void split_fixup(const GemmArgs& p, int b, int m0, int n0, unsigned* 
     for (int g = threadIdx.x; g < BM * G4; g += NT) {
         const int row = m0 + g / G4, col = n0 + (g % G4) * 4;
         if (row >= p.M || col >= p.N) continue;
-        const int64_t e = (int64_t)b * mn + (int64_t)row * p.N + col;
+        const int64_t e = (int64_t)b * mn + (int64_t)row * p.np + col;
         f32x4 v = ld(e);
         // four planes' loads in flight before their adds (still in split order)
         int z = 1;

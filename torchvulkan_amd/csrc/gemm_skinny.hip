@@ -10,8 +10,9 @@
 // columns against the 16 rows of A. B stored k-contiguous ([N][K], a transposed
 // weight view) is loaded straight into MFMA operands; B stored n-contiguous
 // ([K][N]) is written to a wave-private LDS tile as it arrives and read back
-// along k. It runs the layouts without 16-byte rows, and n-contiguous B where
-// the ring below does not apply.
+// along k. It runs the layouts without 16-byte rows, n-contiguous B where the
+// ring below does not apply, and k-contiguous B where its ring does not pay
+// (kring_pays).
 //
 // B n-contiguous with 16-byte aligned rows ([K][N], the C5 layout) takes a
 // second kernel, gemm16_skinny_ring: workgroups of 8 waves own 128 columns
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
             for (int r = 0; r < 4; ++r) {
                 const int row = m * 16 + g * 4 + r;
                 if (row >= p.M) continue;
-                const int64_t pi = (((int64_t)z * p.batch + b) * p.M + row) * p.N + n;
+                const int64_t pi = (((int64_t)z * p.batch + b) * p.M + row) * p.np + n;
                 if (p.split > 1 && p.tile_count) part_store(part_rsrc(p), pi, acc[m][r]);
                 else if (p.split > 1) p.part[pi] = acc[m][r];
                 else store_out<DT, true>(p, b, row, n, acc[m][r]);
@@ -434,10 +435,37 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
                                                    reinterpret_cast<int*>(lds_raw));
 }
 
+// The range where the ring leads the kernels that take these products without
+// it (up to 16 rows gemm_skinny_kernel, above it the 64x64 tiles and from
+// K = 2048 the split 128x128 tiles). It runs one workgroup a CU, whose stages
+// are 256 k, so it wants about one round of workgroups and a whole stage:
+//   - M <= 16, K >= 256 (8 rows, 32 x 2048 x 64: 1.15x the other kernel's
+//     time, K = 128 1.07x, 256 0.92x), and up to 384 workgroups or K >= 1536
+//     (4 x 128256 x 256 1.22x, x 1024 1.03x, x 1536 0.87x).
+//   - above, K >= 8 M: a stage does the products of whole 16-row blocks, 4 of
+//     them from 33 rows (64 x 4096 x 256 1.12x, x 512 0.99x; 32 x 4096 x 128
+//     0.94x, 256 0.81x).
+//   - at most one round of workgroups, 224 with 4 row blocks (64 x 20000 x
+//     1024, 313 of them, 1.43x; batch 64 of 64 x 512 x 1000 1.29x; 256 of them
+//     1.07x) except over one long wide weight, where the tiles starve too (32
+//     x 32000 x 5000 0.66x).
+//   - batches split K less well: from K = 2048, where the tiles split too, up
+//     to 64 workgroups (batch 16 of 32 x 512 x 8192, 128 of them, 1.17x; 4 of
+//     32 x 1000 x 4096 0.81x).
+bool kring_pays(const GemmArgs& p) {
+    const int64_t wgs = (int64_t)((p.N + SKR_NB - 1) / SKR_NB) * p.batch;
+    if (p.M <= 16) return p.K >= 256 && (wgs <= 384 || p.K >= 1536);
+    if (p.M > (p.K < 8192 ? 64 : 32) || p.K < 8 * p.M) return false;
+    if (p.batch > 1 && p.K >= 2048 && wgs > 64) return false;
+    if (p.M <= 32) return wgs <= 256 || (p.batch == 1 && p.K >= 4096);
+    return wgs <= 224;
+}
+
 bool kring_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
+    if (!kring_pays(p)) return false;
     auto al16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
     if (!b_kmajor || !vec || !al16(p.a) || !al16(p.b) || p.sa[2] != 1 || p.sb[1] != 1) return false;
-    if (p.M > 64 || p.K % 8 != 0 || (p.M > 1 && p.sa[1] % 8 != 0) || (p.N > 1 && p.sb[2] % 8 != 0)) return false;
+    if (p.K % 8 != 0 || (p.M > 1 && p.sa[1] % 8 != 0) || (p.N > 1 && p.sb[2] % 8 != 0)) return false;
     if (p.batch > 1 && (p.sa[0] % 8 != 0 || p.sb[0] % 8 != 0)) return false;
     if (p.bh > 1 && (p.sa_h % 8 != 0 || p.sb_h % 8 != 0)) return false;
     return true;
@@ -452,12 +480,18 @@ KringShape kring_shape(const GemmArgs& p) {
     KringShape r;
     r.strips = (p.N + SKR_NB - 1) / SKR_NB;
     const int stages = (p.K + SKR_KST - 1) / SKR_KST;
-    // (the fixup and the second launch read 16-byte rows of partials)
-    const int64_t want = p.N % 4 == 0 ? std::min<int64_t>(256 / ((int64_t)r.strips * p.batch), stages / 4) : 1;
+    const int64_t want = std::min<int64_t>(256 / ((int64_t)r.strips * p.batch), stages / 4);
     const int per = want > 1 ? (int)((stages + want - 1) / want) : stages;
     r.chunk = per * SKR_KST;
     r.split = (stages + per - 1) / per;
     return r;
+}
+
+// Bytes of the partials of `split` chunks: rows of N rounded up to 4, which the
+// fixup and the second launch read 16 bytes at a time.
+int kring_pitch(const GemmArgs& p) { return (p.N + 3) / 4 * 4; }
+size_t kring_part_bytes(const GemmArgs& p, int split) {
+    return split > 1 ? (size_t)split * p.batch * p.M * kring_pitch(p) * 4 : 0;
 }
 
 template <int DT>
@@ -484,7 +518,7 @@ bool skinny_applies(int64_t M, int64_t N, int64_t K, int64_t batch) {
 }
 
 bool skinny_wide_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
-    return p.M > 16 && p.M <= (p.K < 8192 ? 64 : 32) && skinny_applies(16, p.N, p.K, p.batch) && kring_applies(p, b_kmajor, vec);
+    return p.M > 16 && skinny_applies(16, p.N, p.K, p.batch) && kring_applies(p, b_kmajor, vec);
 }
 
 const char* skinny_name(const GemmArgs& p, bool b_kmajor, bool vec) {
@@ -493,10 +527,7 @@ const char* skinny_name(const GemmArgs& p, bool b_kmajor, bool vec) {
 }
 
 size_t skinny_scratch_bytes(const GemmArgs& p, bool b_kmajor, bool vec) {
-    if (kring_applies(p, b_kmajor, vec)) {
-        const int split = kring_shape(p).split;
-        return split > 1 ? (size_t)split * p.batch * p.M * p.N * 4 : 0;
-    }
+    if (kring_applies(p, b_kmajor, vec)) return kring_part_bytes(p, kring_shape(p).split);
     if (!ring_applies(p, b_kmajor, vec)) return 0;
     const int split = ring_splits(p);
     return split > 1 ? (size_t)split * p.batch * p.M * p.N * 4 : 0;
@@ -506,7 +537,7 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
     if (kring_applies(p, b_kmajor, vec)) {
         GemmArgs q = p;
         const KringShape ks = kring_shape(p);
-        q.np = q.N;
+        q.np = kring_pitch(p);
         q.split = ks.split;
         q.k_chunk = ks.chunk;
         Scratch scratch;
@@ -516,7 +547,7 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
             // scratch also under capture: a captured call does so where the stream's pool holds an idle buffer, and
             // sums the partials in a second launch (unsplit, few strips leave most CUs idle: bfloat16 33 x 8000 x 256
             // 29.1 us, 10.9 on split tiles, 9.7 so).
-            const size_t bytes = (size_t)q.split * p.batch * p.M * p.N * 4;
+            const size_t bytes = kring_part_bytes(p, q.split);
             const bool fits = bytes < (size_t)1 << 31, usable = scratch_usable(s);
             const bool idle = !usable && p.M > 16 && p.K >= 2048 && s != hipStreamPerThread;
             q.part = nullptr;
@@ -562,10 +593,10 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
     dim3 grid(strips, 1, p.batch);
 #define TVK_SK(D, BKM, V) hipLaunchKernelGGL((gemm_skinny_kernel<D, BKM, V>), grid, dim3(64 * SK_NW), 0, s, p)
     if (dtype == TVK_F16) {
-        if (b_kmajor) TVK_SK(TVK_F16, true, false);   // (with 16-byte rows: the ring)
+        if (b_kmajor) { if (vec) TVK_SK(TVK_F16, true, true); else TVK_SK(TVK_F16, true, false); }
         else { if (vec) TVK_SK(TVK_F16, false, true); else TVK_SK(TVK_F16, false, false); }
     } else {
-        if (b_kmajor) TVK_SK(TVK_BF16, true, false);
+        if (b_kmajor) { if (vec) TVK_SK(TVK_BF16, true, true); else TVK_SK(TVK_BF16, true, false); }
         else { if (vec) TVK_SK(TVK_BF16, false, true); else TVK_SK(TVK_BF16, false, false); }
     }
 #undef TVK_SK
