@@ -64,8 +64,8 @@ def test_views_batches_and_epilogue(gpu, m):
 
 @pytest.mark.parametrize("m", [16, 64])
 def test_noalloc_and_capture(gpu, m):
-    # without scratch of the pool: the allocation-free entry point sums in a second launch, a captured call whose
-    # stream has no idle scratch runs unsplit
+    # without scratch of the pool: the allocation-free entry point sums in a second launch above 16 rows, up to them,
+    # and in a captured call whose stream has no idle scratch, a workgroup takes the chunks of K in turn
     dtype = torch.bfloat16
     x, w = operands(m, 512, 8192 if m == 16 else 4096, dtype, 11)
     want = x.double() @ w.double().t()
@@ -109,3 +109,50 @@ def test_capture_on_a_warm_stream(gpu, m, n, k):
         _abi.gemm(xd, wd.t(), e)
         torch.cuda.synchronize()
         assert torch.equal(c.cpu().double(), want) and torch.equal(e, c)
+
+
+# real values whose sums round: the split call (K in chunks over workgroups), the allocation-free entry point and a
+# captured call on a stream without idle scratch give the same bits; biases and activations in either epilogue
+@pytest.mark.parametrize("m", [1, 7, 16, 17, 40, 64])
+@pytest.mark.parametrize("n,k", [(64, 2048), (250, 4104), (1000, 6000), (512, 1800)])
+def test_same_bits_without_partials(gpu, m, n, k):
+    dtype = torch.bfloat16 if n % 4 else torch.float16
+    g = torch.Generator().manual_seed(m + n)
+    x, w = torch.randn((m, k), generator=g).to(dtype).to(DEV), torch.randn((n, k), generator=g).to(dtype).to(DEV)
+    kw = {"bias": torch.randn((n,), generator=g).to(dtype).to(DEV), "alpha": 0.5, "beta": 2.0, "activation": _abi.TVK_ACT_GELU}
+    for kw in ({}, kw):
+        want, got, captured = (torch.full((m, n), 7, dtype=dtype, device=DEV) for _ in range(3))
+        _abi.gemm(x, w.t(), want, **kw)
+        _abi.gemm_noalloc(x, w.t(), got, **kw)
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            _abi.gemm(x, w.t(), captured, **kw)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(captured, want)
+
+
+# the allocation-free entry point up to 16 rows uses none of the array its calls share: calls that overlap, replayed
+# from two graphs on two streams, are independent
+def test_noalloc_overlapping_calls(gpu):
+    m, n, k, calls = 16, 1024, 8192, 20
+    x, w = operands(m, n, k, torch.bfloat16, 3)
+    xs, wd = [(x * (i + 1)).to(DEV) for i in range(2)], w.to(DEV)
+    outs = [torch.empty((calls, m, n), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    graphs, streams = [], [torch.cuda.Stream() for _ in range(2)]
+    for j, st in enumerate(streams):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[j], stream=st):
+            for i in range(calls):
+                _abi.gemm_noalloc(xs[j], wd.t(), outs[j][i])
+    want = x.double() @ w.double().t()
+    for _ in range(5):
+        for j, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                outs[j].zero_()
+                graphs[j].replay()
+        torch.cuda.synchronize()
+        for j in range(2):
+            ok = (outs[j].cpu().double() == (j + 1) * want).flatten(1).all(dim=1)
+            assert ok.all(), f"stream {j}: {int((~ok).sum())} of {calls} calls differ"

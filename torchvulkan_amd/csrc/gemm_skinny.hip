@@ -312,7 +312,8 @@ int ring_splits(const GemmArgs& p) {
 //   - K is split between workgroups up to about one per CU in chunks of at
 //     least four stages (the exchange costs about 1.5 us: 7 x 1000 -> 500 takes
 //     5.2 us whole, 6.2 in two), summed by the last workgroup of a strip
-//     (split_fixup) or a second launch.
+//     (split_fixup) or a second launch; without memory for partials a
+//     workgroup takes a strip's chunks in turn (SERIAL).
 //   - MF 16-row blocks of A: up to 64 rows (4096 -> 14336: 24.3 us for 32 rows,
 //     31.7 for 64; the split 128 x 128 ring took 33.1 and 36.8). Above 32 rows A
 //     weighs as much as B in the ring, and from K = 8192 the 128 x 128 tiles
@@ -326,22 +327,36 @@ constexpr int SKR_B = SR_NW * 16 * SKR_K * 2;   // B bytes per stage: 32 KB, 4 K
 // LDS bytes of a stage (MF 16-row blocks of A) and ring depth in 160 KB
 constexpr int kring_stage(int mf) { return SKR_B + mf * SKR_KG * 4096; }
 constexpr int kring_depth(int mf) { return std::min(4, 160 * 1024 / kring_stage(mf)); }
+// and of the k halves' exchange, beside a ring of at most 3 stages where it recurs (SERIAL)
+constexpr int kring_red(int mf) { return SR_NW / SKR_KG * mf * 1024; }
 
-template <int DT, int MF>
+// SERIAL: one workgroup takes a strip's K chunks one after another, for calls
+// without memory for partials. It adds the chunks' sums in chunk order, the
+// additions of split_fixup, so a call gives the same bits either way.
+template <int DT, int MF, bool SERIAL>
 __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs p) {
     constexpr int CG = SR_NW / SKR_KG;   // 16-column groups
-    constexpr int NS = kring_depth(MF), STB = kring_stage(MF);
+    constexpr int NS = SERIAL ? std::min(3, kring_depth(MF)) : kring_depth(MF), STB = kring_stage(MF);
     constexpr int AL = 4 * MF * SKR_KG / SR_NW;   // A loads per wave
     static_assert(AL * SR_NW == 4 * MF * SKR_KG, "whole loads");
-    __shared__ __attribute__((aligned(1024))) char lds_raw[NS * STB];
+    static_assert(NS * STB + (SERIAL ? kring_red(MF) : 0) <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) char lds_raw[NS * STB + (SERIAL ? kring_red(MF) : 0)];
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TVK_LDS char*)lds_raw);
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int cg = wave % CG, kg = wave / CG;
     const int n0 = blockIdx.x * SKR_NB, z = blockIdx.y, b = blockIdx.z;
-    const int kb = p.split > 1 ? z * p.k_chunk : 0;
-    const int kend = p.split > 1 ? min(p.K, kb + p.k_chunk) : p.K;
+    const bool split = !SERIAL && p.split > 1;
+    const int kb = split ? z * p.k_chunk : 0;
+    const int kend = split ? min(p.K, kb + p.k_chunk) : p.K;
     const int nk = (kend - kb + SKR_KST - 1) / SKR_KST;
-    const int rot = p.sb[2] % 2048 == 0 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)nk) : 0;
+    const int per = SERIAL ? p.k_chunk / SKR_KST : nk;   // stages of a chunk
+    // the stage that the s-th load brings: a chunk's stages from its workgroup's first one round
+    auto stage_at = [&](int s) {
+        const int c0 = SERIAL ? s / per * per : 0, n = SERIAL ? min(per, nk - c0) : nk;
+        const int rot = p.sb[2] % 2048 == 0 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)n) : 0;
+        const int i = s - c0 + rot;
+        return c0 + (i >= n ? i - n : i);
+    };
 
     const char* A = reinterpret_cast<const char*>(p.a) + a_boff(p, b) * 2;
     const char* B = reinterpret_cast<const char*>(p.b) + b_boff(p, b) * 2;
@@ -365,8 +380,7 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
     auto issue = [&](int s) {
         if (s >= nk) return;
         const uint32_t slot = lds0 + (uint32_t)((s % NS) * STB);
-        int ks = s + rot;
-        if (ks >= nk) ks -= nk;
+        const int ks = stage_at(s);
         const int left = p.K - kb - ks * SKR_KST;   // chunks at or past it would read the next row: zeros instead
         const uint32_t step = (uint32_t)(ks * SKR_KST * 2);
 #pragma unroll
@@ -377,9 +391,22 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
             sr_dma16(ra, slot + SKR_B + (uint32_t)((wave * AL + q) * 1024), a_k[q] < left ? a_off[q] + step : kOOB);
     };
 
-    f32x4 acc[MF];
+    f32x4 acc[MF], total[MF];   // (total: SERIAL only)
 #pragma unroll
-    for (int m = 0; m < MF; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int m = 0; m < MF; ++m) acc[m] = total[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    // the second k half's sums onto the first's
+    f32x4* red = reinterpret_cast<f32x4*>(lds_raw + (SERIAL ? NS * STB : 0));
+    auto add_halves = [&]() {
+        if (kg > 0) {
+#pragma unroll
+            for (int m = 0; m < MF; ++m) red[(cg * MF + m) * 64 + lane] = acc[m];
+        }
+        __syncthreads();
+        if (kg == 0) {
+#pragma unroll
+            for (int m = 0; m < MF; ++m) acc[m] += red[(cg * MF + m) * 64 + lane];
+        }
+    };
 #pragma unroll
     for (int s = 0; s < NS - 1; ++s) issue(s);
     const int g = lane / 16, c16 = lane % 16;
@@ -400,19 +427,22 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
                 acc[m] = mfma16<DT>(af, bf, acc[m]);
             }
         }
+        if (SERIAL && ((kt + 1) % per == 0 || kt == nk - 1)) {
+            add_halves();   // (read again after the next stage's barrier at the earliest)
+#pragma unroll
+            for (int m = 0; m < MF; ++m) {
+                total[m] = kt < per ? acc[m] : total[m] + acc[m];
+                acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
     }
     sr_wait<0>();
-    // the second k half's sums onto the first's
     __syncthreads();
-    f32x4* red = reinterpret_cast<f32x4*>(lds_raw);
-    if (kg > 0) {
+    if constexpr (SERIAL) {
 #pragma unroll
-        for (int m = 0; m < MF; ++m) red[(cg * MF + m) * 64 + lane] = acc[m];
-    }
-    __syncthreads();
-    if (kg == 0) {
-#pragma unroll
-        for (int m = 0; m < MF; ++m) acc[m] += red[(cg * MF + m) * 64 + lane];
+        for (int m = 0; m < MF; ++m) acc[m] = total[m];
+    } else {
+        add_halves();
     }
 
     // lane l holds column l % 16 of the wave's 16, rows 16 m + (l / 16) * 4 + r
@@ -425,12 +455,12 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
                 const int row = m * 16 + g * 4 + r;
                 if (row >= p.M) continue;
                 const int64_t pi = (((int64_t)z * p.batch + b) * p.M + row) * p.np + n;
-                if (p.split > 1 && p.tile_count) part_store(part_rsrc(p), pi, acc[m][r]);
-                else if (p.split > 1) p.part[pi] = acc[m][r];
+                if (split && p.tile_count) part_store(part_rsrc(p), pi, acc[m][r]);
+                else if (split) p.part[pi] = acc[m][r];
                 else store_out<DT, true>(p, b, row, n, acc[m][r]);
             }
     }
-    if (p.split > 1 && p.tile_count)
+    if (split && p.tile_count)
         split_fixup<DT, 64 * SR_NW, 16 * MF, SKR_NB>(p, b, 0, n0, p.tile_count + (int64_t)b * gridDim.x + blockIdx.x,
                                                    reinterpret_cast<int*>(lds_raw));
 }
@@ -494,13 +524,27 @@ size_t kring_part_bytes(const GemmArgs& p, int split) {
     return split > 1 ? (size_t)split * p.batch * p.M * kring_pitch(p) * 4 : 0;
 }
 
-template <int DT>
+template <int DT, bool SERIAL>
 void launch_kring(const GemmArgs& q, const KringShape& ks, hipStream_t s) {
-    const dim3 grid(ks.strips, q.split, q.batch), block(64 * SR_NW);
-    if (q.M <= 16) hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 1>), grid, block, 0, s, q);
-    else if (q.M <= 32) hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 2>), grid, block, 0, s, q);
-    else hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 4>), grid, block, 0, s, q);
+    const dim3 grid(ks.strips, SERIAL ? 1 : q.split, q.batch), block(64 * SR_NW);
+    if (q.M <= 16) hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 1, SERIAL>), grid, block, 0, s, q);
+    else if (q.M <= 32) hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 2, SERIAL>), grid, block, 0, s, q);
+    else hipLaunchKernelGGL((gemm_skinny_kring_kernel<DT, 4, SERIAL>), grid, block, 0, s, q);
 }
+
+// The kernel, and where K is split into a pool's or the caller's partials
+// without counters their reduction.
+template <int DT>
+void launch_kring_all(const GemmArgs& q, const KringShape& ks, hipStream_t s) {
+    if (q.split > 1 && !q.part) return launch_kring<DT, true>(q, ks, s);
+    launch_kring<DT, false>(q, ks, s);
+    if (q.split > 1 && !q.tile_count) launch_split_reduce<DT>(q, s);
+}
+
+// Whether a call that may not share memory with others, or must not allocate,
+// splits K over workgroups all the same: up to 16 rows, and below K = 2048,
+// such products have always been summed without partials.
+bool kring_shared_split(const GemmArgs& p) { return p.M > 16 && p.K >= 2048; }
 
 bool ring_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
     if (b_kmajor || !vec) return false;
@@ -527,7 +571,7 @@ const char* skinny_name(const GemmArgs& p, bool b_kmajor, bool vec) {
 }
 
 size_t skinny_scratch_bytes(const GemmArgs& p, bool b_kmajor, bool vec) {
-    if (kring_applies(p, b_kmajor, vec)) return kring_part_bytes(p, kring_shape(p).split);
+    if (kring_applies(p, b_kmajor, vec)) return kring_shared_split(p) ? kring_part_bytes(p, kring_shape(p).split) : 0;
     if (!ring_applies(p, b_kmajor, vec)) return 0;
     const int split = ring_splits(p);
     return split > 1 ? (size_t)split * p.batch * p.M * p.N * 4 : 0;
@@ -541,29 +585,23 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
         q.split = ks.split;
         q.k_chunk = ks.chunk;
         Scratch scratch;
-        if (q.split > 1 && !part) {
-            // A call without scratch of its own (capture: its counters must not be touched and it must not allocate; no
-            // memory) runs unsplit, as up to 16 rows always did. Above, the tiled plans split from K = 2048 and lease
-            // scratch also under capture: a captured call does so where the stream's pool holds an idle buffer, and
-            // sums the partials in a second launch (unsplit, few strips leave most CUs idle: bfloat16 33 x 8000 x 256
-            // 29.1 us, 10.9 on split tiles, 9.7 so).
+        q.part = nullptr;   // (without partials a workgroup takes a strip's chunks one after another)
+        if (q.split > 1 && part) {   // the caller's memory, which its calls on other streams share
+            if (kring_shared_split(p)) q.part = part;
+        } else if (q.split > 1) {
+            // Capture must not touch the counters and must not allocate. Above 16 rows the tiled plans split from K =
+            // 2048 and lease scratch also under capture: a captured call does so where the stream's pool holds an idle
+            // buffer, and sums the partials in a second launch (in one workgroup a strip few strips leave most CUs
+            // idle: bfloat16 33 x 8000 x 256 29.1 us, 10.9 on split tiles, 9.7 so).
             const size_t bytes = kring_part_bytes(p, q.split);
             const bool fits = bytes < (size_t)1 << 31, usable = scratch_usable(s);
-            const bool idle = !usable && p.M > 16 && p.K >= 2048 && s != hipStreamPerThread;
-            q.part = nullptr;
+            const bool idle = !usable && kring_shared_split(p) && s != hipStreamPerThread;
             if (fits && usable) q.part = static_cast<float*>(scratch.get(bytes, s));
             else if (fits && idle) q.part = static_cast<float*>(scratch.get_idle(bytes, s));
             if (q.part) q.tile_count = split_counters(s, (int64_t)ks.strips * p.batch);
-            else q.split = 1;
-        } else {
-            q.part = part;
         }
-        if (dtype == TVK_F16) launch_kring<TVK_F16>(q, ks, s);
-        else launch_kring<TVK_BF16>(q, ks, s);
-        if (q.split > 1 && !q.tile_count) {
-            if (dtype == TVK_F16) launch_split_reduce<TVK_F16>(q, s);
-            else launch_split_reduce<TVK_BF16>(q, s);
-        }
+        if (dtype == TVK_F16) launch_kring_all<TVK_F16>(q, ks, s);
+        else launch_kring_all<TVK_BF16>(q, ks, s);
         return hipGetLastError();
     }
     if (ring_applies(p, b_kmajor, vec)) {
