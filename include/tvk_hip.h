@@ -26,7 +26,15 @@
  *     threads, other streams) get other buffers; buffers are freed only after
  *     the device has drained (on growth, allocation failure or
  *     tvk_empty_cache). Calls may therefore come from any thread and any
- *     stream; the caller orders only its own tensors.
+ *     stream; the caller orders only its own tensors. A call under HIP graph
+ *     capture gets memory of the graph's own (2 MiB or more a stream of the
+ *     capture), allocated at capture and given back to the pool when the graph
+ *     and everything instantiated from it are destroyed: its replays run on any
+ *     stream, beside any other call. Two executables instantiated from one
+ *     graph share that memory and must not run at the same time. Attention of
+ *     at most 16 queries and few-row products with a k-contiguous weight of up
+ *     to 16 rows need none under capture: the first takes the keys, the second
+ *     a strip's chunks of K, in one workgroup each.
  */
 #ifndef TVK_HIP_H
 #define TVK_HIP_H
@@ -464,11 +472,13 @@ tvk_status tvk_attention_bwd(const tvk_attention_bwd_desc* desc);
  *
  * Scratch: split-K partials and repacked operands come from a per-device pool
  * of stream-affine buffers (freed by tvk_empty_cache after a drain). The
- * M <= 16 streaming kernel reduces its split-K partials in the same launch,
- * counting finished workgroups in a 64 KB array per stream (allocated at the
- * stream's first such product, kept until the process ends, at most 32
- * streams a device); launches under graph capture, on hipStreamPerThread and
- * on further streams use a second reduction launch instead. */
+ * streaming kernels of few rows (up to 16, with a k-contiguous B up to 64)
+ * reduce their split-K partials in the same launch, counting finished
+ * workgroups in a 64 KB array per stream (allocated at the stream's first such
+ * product, kept until the process ends, at most 32 streams a device); launches
+ * under graph capture, on hipStreamPerThread and on further streams use a
+ * second reduction launch, or sum the chunks of K in one workgroup, with the
+ * same bits. */
 /* tvk_gemm_desc.flags */
 #define TVK_GEMM_EXACT 1u   /* every dtype in the reference SIMD tile's order:
                                float32 operands, fmaf over k = 0..K-1 in

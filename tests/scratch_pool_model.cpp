@@ -7,9 +7,12 @@
 //      its successive holders);
 //   3. two holders never share a buffer;
 //   4. the hot path (a lease for a stream that has a large enough idle
-//      buffer) neither allocates nor drains the device.
+//      buffer) neither allocates nor drains the device;
+//   5. a buffer that a captured call used is its graph's: launches of the graph
+//      use it on any stream, and until the graph is gone no other call leases
+//      it and nothing frees it.
 // Scenarios: same-stream reuse, several streams, growth while another lease is
-// held, out-of-memory recovery, and a multi-threaded stress run.
+// held, out-of-memory recovery, captured calls, and a multi-threaded stress run.
 // Prints "ok" and exits 0 on success; any violation aborts with a message.
 #include "scratch_pool.h"
 
@@ -69,6 +72,12 @@ struct Model {
         for (auto& kv : queue) kv.second.clear();
         ++drains;
     }
+    struct Capture {
+        uint64_t id;
+        struct Graph* graph;
+    };
+    void* alloc_captured(size_t bytes) { return alloc(bytes); }
+    inline bool keep(const Capture& c, std::atomic<bool>* returned);
 
     // ---- simulation ----
     void use(void* p, int s) {
@@ -86,6 +95,34 @@ struct Model {
 };
 
 typedef tvk::ScratchPool<Model> Pool;
+
+// A graph: the buffers its kernels use, and what it tells when it is gone.
+struct Graph {
+    std::vector<void*> uses;
+    std::vector<std::atomic<bool>*> keeps;
+    bool refuse = false;
+    void launch(Model& m, int s) {
+        std::lock_guard<std::recursive_mutex> lk(m.mu);
+        for (void* p : uses) {
+            CHECK(m.live.count(p) == 1, "a graph launch uses a freed buffer");
+            CHECK(m.home.count(p) == 0, "a graph's buffer was used by an eager call");
+            m.queue[s].push_back(p);
+        }
+    }
+    void destroy() {
+        for (auto* r : keeps) r->store(true);
+        uses.clear();
+        keeps.clear();
+    }
+};
+bool Model::keep(const Capture& c, std::atomic<bool>* returned) {
+    if (c.graph->refuse) {
+        returned->store(true);
+        return false;
+    }
+    c.graph->keeps.push_back(returned);
+    return true;
+}
 
 void same_stream_reuse() {
     Model m;
@@ -167,6 +204,72 @@ void out_of_memory() {
     CHECK(m.live.empty(), "every buffer freed");
 }
 
+// One captured call on stream s: a lease, a kernel in the graph, the lease's end.
+void* captured_call(Pool& pool, Graph& g, uint64_t id, size_t bytes, int s) {
+    auto* b = pool.acquire_captured(bytes, s, Model::Capture{id, &g});
+    if (!b) return nullptr;
+    CHECK(b->bytes >= bytes, "a captured call's buffer is large enough");
+    void* p = b->ptr;
+    g.uses.push_back(p);
+    pool.release(b);
+    return p;
+}
+
+void captured_calls() {
+    Model m;
+    Pool pool(m, 1024);
+    auto eager = [&](size_t bytes, int s) {
+        auto* b = pool.acquire(bytes, s);
+        CHECK(b, "an eager lease");
+        m.use(b->ptr, s);
+        pool.release(b);
+    };
+    eager(100, 1);   // an idle buffer that the capture must not take: its kernels may still run
+    Graph g, h;
+    void* a = captured_call(pool, g, 7, 100, 1);
+    CHECK(a && m.home.count(a) == 0, "a captured call gets a buffer that no eager call used");
+    CHECK(captured_call(pool, g, 7, 200, 1) == a, "calls of one capture on one stream share a buffer");
+    CHECK(captured_call(pool, g, 7, 200, 2) != a, "a second stream of the capture has its own");
+    CHECK(captured_call(pool, h, 8, 200, 1) != a, "a second graph of the stream has its own");
+    void* big = captured_call(pool, g, 7, 5 << 20, 1);
+    CHECK(big != a, "a larger request gets a larger buffer");
+    CHECK(pool.captured_count() == 4, "four buffers belong to the graphs");
+    // eager growth on the capture's stream, a launch on another stream, a trim while it is pending
+    eager(1 << 20, 1);
+    eager(6 << 20, 1);
+    g.launch(m, 3);
+    h.launch(m, 4);
+    pool.trim();
+    g.launch(m, 1);
+    eager(100, 1);
+    m.sync_device();
+    // an allocation failure gives back what is idle, not the graphs' buffers
+    m.budget = m.in_use + 1000;
+    CHECK(pool.acquire(size_t(1) << 30, 5) == nullptr, "no memory");
+    m.budget = size_t(1) << 40;
+    g.launch(m, 2);
+    m.sync_device();
+    // a graph that is gone gives its buffers to later captures, and to trim
+    g.destroy();
+    CHECK(pool.captured_count() == 1, "only the second graph's buffer is left");
+    Graph k;
+    const long allocs = m.allocs;
+    void* again = captured_call(pool, k, 9, 100, 6);
+    CHECK(m.allocs == allocs && again, "a later capture takes a buffer of a graph that is gone");
+    k.launch(m, 6);
+    pool.trim();
+    CHECK(m.live.count(again) == 1, "and keeps it");
+    m.sync_device();
+    // a graph that cannot be told: no lease, and the memory is not lost
+    Graph r;
+    r.refuse = true;
+    CHECK(captured_call(pool, r, 10, 100, 1) == nullptr && captured_call(pool, r, 10, 100, 1) == nullptr, "refused");
+    h.destroy();
+    k.destroy();
+    pool.trim();
+    CHECK(m.live.empty() && m.allocs == m.frees, "every buffer freed once");
+}
+
 void threads() {
     Model m;
     Pool pool(m, 256);
@@ -207,6 +310,7 @@ int main() {
     streams_keep_their_buffers();
     grow_while_held();
     out_of_memory();
+    captured_calls();
     threads();
     std::printf("ok\n");
     return 0;

@@ -589,16 +589,13 @@ hipError_t launch_skinny(int dtype, const GemmArgs& p, bool b_kmajor, bool vec, 
         if (q.split > 1 && part) {   // the caller's memory, which its calls on other streams share
             if (kring_shared_split(p)) q.part = part;
         } else if (q.split > 1) {
-            // Capture must not touch the counters and must not allocate. Above 16 rows the tiled plans split from K =
-            // 2048 and lease scratch also under capture: a captured call does so where the stream's pool holds an idle
-            // buffer, and sums the partials in a second launch (in one workgroup a strip few strips leave most CUs
-            // idle: bfloat16 33 x 8000 x 256 29.1 us, 10.9 on split tiles, 9.7 so).
+            // A captured call takes memory of the graph's own where the tiled plans, which split from K = 2048 above 16
+            // rows, take it too, and sums the partials in a second launch (in one workgroup a strip few strips leave
+            // most CUs idle: bfloat16 33 x 8000 x 256 29.1 us, 10.9 on split tiles, 9.7 so).
             const size_t bytes = kring_part_bytes(p, q.split);
-            const bool fits = bytes < (size_t)1 << 31, usable = scratch_usable(s);
-            const bool idle = !usable && kring_shared_split(p) && s != hipStreamPerThread;
-            if (fits && usable) q.part = static_cast<float*>(scratch.get(bytes, s));
-            else if (fits && idle) q.part = static_cast<float*>(scratch.get_idle(bytes, s));
-            if (q.part) q.tile_count = split_counters(s, (int64_t)ks.strips * p.batch);
+            if (bytes < (size_t)1 << 31 && (scratch_usable(s) || (kring_shared_split(p) && s != hipStreamPerThread)))
+                q.part = static_cast<float*>(scratch.get(bytes, s));
+            if (q.part) q.tile_count = split_counters(s, (int64_t)ks.strips * p.batch);   // (NULL under capture)
         }
         if (dtype == TVK_F16) launch_kring_all<TVK_F16>(q, ks, s);
         else launch_kring_all<TVK_BF16>(q, ks, s);

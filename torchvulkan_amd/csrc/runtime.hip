@@ -115,7 +115,56 @@ struct HipScratchBackend {
     }
     void free(void* p) { On on(device); (void)hipFree(p); }
     void sync_device() { On on(device); (void)hipDeviceSynchronize(); }
+
+    struct Capture {
+        uint64_t id;
+        hipGraph_t graph;
+    };
+    // (a capture in the global or thread-local mode refuses hipMalloc, and is ended by it, unless the thread steps out)
+    void* alloc_captured(size_t bytes) {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        void* p = alloc(bytes);
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        return p;
+    }
+    // A user object of the graph: the runtime destroys it with the last of the graph, its clones and its executables,
+    // after their launches. (The callback may run on a thread of the runtime, inside its locks: it only sets the flag.)
+    bool keep(const Capture& c, std::atomic<bool>* returned) {
+        hipUserObject_t obj = nullptr;
+        if (hipUserObjectCreate(&obj, returned, [](void* p) { static_cast<std::atomic<bool>*>(p)->store(true); }, 1,
+                                hipUserObjectNoDestructorSync) != hipSuccess) {
+            (void)hipGetLastError();
+            returned->store(true);
+            return false;
+        }
+        if (hipGraphRetainUserObject(c.graph, obj, 1, hipGraphUserObjectMove) == hipSuccess) return true;
+        (void)hipGetLastError();
+        (void)hipUserObjectRelease(obj, 1);   // (sets the flag)
+        return false;
+    }
 };
+
+// The capture that `stream` is part of, if it is being captured.
+bool capture_of(hipStream_t stream, HipScratchBackend::Capture& c) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (st != hipStreamCaptureStatusActive) return false;
+    unsigned long long id = 0;
+    c.graph = nullptr;
+    if (hipStreamGetCaptureInfo_v2(stream, &st, &id, &c.graph, nullptr, nullptr) != hipSuccess || !c.graph) {
+        (void)hipGetLastError();
+        return false;
+    }
+    c.id = id;
+    return true;
+}
 
 struct DeviceScratch {
     HipScratchBackend backend;
@@ -134,16 +183,13 @@ DeviceScratch* device_scratch(int device) {
 
 }  // namespace
 
-void* Scratch::get(size_t bytes, hipStream_t stream) { return lease(bytes, stream, false); }
-
-void* Scratch::get_idle(size_t bytes, hipStream_t stream) { return lease(bytes, stream, true); }
-
-void* Scratch::lease(size_t bytes, hipStream_t stream, bool idle_only) {
+void* Scratch::get(size_t bytes, hipStream_t stream) {
     release();
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return nullptr;
     auto& pool = device_scratch(dev)->pool;
-    auto* buf = idle_only ? pool.acquire_idle(bytes, stream) : pool.acquire(bytes, stream);
+    HipScratchBackend::Capture c;
+    auto* buf = capture_of(stream, c) ? pool.acquire_captured(bytes, stream, c) : pool.acquire(bytes, stream);
     if (!buf) return nullptr;
     lease_ = buf;
     device_ = dev;

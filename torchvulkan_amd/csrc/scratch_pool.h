@@ -13,13 +13,21 @@
 //   - buffers are freed only on a slow path (a request larger than every idle
 //     buffer of its stream, an allocation failure, trim), after the whole
 //     device has drained, so no kernel of any stream can still use them; held
-//     buffers are never freed.
+//     buffers are never freed;
+//   - a captured call's kernels run again whenever its graph is launched, on
+//     any stream, long after its lease has ended. Its buffer therefore belongs
+//     to the graph: it is leased again only to later calls of the same capture
+//     on the same stream (which the graph orders behind it), and neither leased
+//     to any other call nor freed before the graph and everything instantiated
+//     from it are gone, which the backend reports through `returned`.
 // The logic is independent of HIP: the backend supplies allocation and the
 // device-wide wait, so the ownership rules can be exercised on the CPU with a
 // model backend.
 #pragma once
 
+#include <atomic>
 #include <cstddef>
+#include <cstdint>
 #include <memory>
 #include <mutex>
 #include <vector>
@@ -31,6 +39,12 @@ namespace tvk {
 //   void* alloc(size_t bytes);    nullptr when out of memory
 //   void free(void* p);
 //   void sync_device();           blocks the host until every stream's work has run
+//   typedef ... Capture;          a capture in progress, with a nonzero `id` of its own
+//   void* alloc_captured(size_t bytes);   alloc, during a capture
+//   bool keep(const Capture& c, std::atomic<bool>* returned);
+//                                 has *returned set once the graph that c builds, and all that is
+//                                 made of it, is gone and has run; false: the graph cannot be told
+//                                 (*returned is set all the same, now or soon)
 template <class B>
 class ScratchPool {
 public:
@@ -41,6 +55,9 @@ public:
         size_t bytes = 0;
         Stream stream{};
         bool held = false;
+        uint64_t capture = 0;              // the capture whose graph owns it, 0: none
+        std::atomic<bool> returned{false};   // that graph is gone
+        bool lendable() const { return !held && capture == 0; }
     };
 
     explicit ScratchPool(B& backend, size_t min_bytes = size_t(16) << 20) : b_(backend), min_bytes_(min_bytes) {}
@@ -55,7 +72,7 @@ public:
         bool small_idle = false;
         for (auto& up : bufs_) {
             Buffer* b = up.get();
-            if (b->held || !(b->stream == s)) continue;
+            if (!b->lendable() || !(b->stream == s)) continue;
             if (b->bytes < bytes) {
                 small_idle = true;
                 continue;
@@ -83,16 +100,44 @@ public:
         return pick;
     }
 
-    // An idle buffer of this stream that is large enough, or nullptr: allocates and frees nothing.
-    Buffer* acquire_idle(size_t bytes, Stream s) {
+    // The same for a call that is being captured: a buffer of the graph's own.
+    Buffer* acquire_captured(size_t bytes, Stream s, const typename B::Capture& c) {
         std::lock_guard<std::mutex> lk(mu_);
         Buffer* pick = nullptr;
+        Buffer* spare = nullptr;   // of a graph that is gone
+        size_t largest = 0;
         for (auto& up : bufs_) {
             Buffer* b = up.get();
-            if (b->held || !(b->stream == s) || b->bytes < bytes) continue;
-            if (!pick || b->bytes < pick->bytes) pick = b;
+            if (b->held || b->capture == 0) continue;
+            if (b->capture == c.id && b->stream == s && !b->returned) {
+                if (b->bytes > largest) largest = b->bytes;
+                if (b->bytes >= bytes && (!pick || b->bytes < pick->bytes)) pick = b;
+            } else if (b->returned && b->bytes >= bytes && (!spare || b->bytes < spare->bytes)) {
+                spare = b;
+            }
         }
-        if (pick) pick->held = true;
+        if (!pick) {
+            std::unique_ptr<Buffer> nb;
+            if (spare) {
+                pick = spare;
+            } else {
+                // the graph's earlier buffers stay with it: at least twice their size, so that there are few
+                size_t sz = bytes > 2 * largest ? bytes : 2 * largest;
+                sz = (sz + kCapturedGrain - 1) / kCapturedGrain * kCapturedGrain;
+                nb.reset(new Buffer());
+                nb->ptr = b_.alloc_captured(sz);
+                if (!nb->ptr) return nullptr;
+                nb->bytes = sz;
+                pick = nb.get();
+            }
+            pick->stream = s;
+            pick->returned = false;
+            const bool kept = b_.keep(c, &pick->returned);
+            pick->capture = kept ? c.id : kNoGraph;
+            if (nb) bufs_.push_back(std::move(nb));
+            if (!kept) return nullptr;
+        }
+        pick->held = true;
         return pick;
     }
 
@@ -103,7 +148,7 @@ public:
         buf->held = false;
     }
 
-    // Frees every idle buffer (held buffers stay).
+    // Frees every idle buffer (held buffers and those of graphs stay).
     void trim() {
         std::lock_guard<std::mutex> lk(mu_);
         retire_idle_locked([](const Buffer&) { return true; });
@@ -122,6 +167,14 @@ public:
         return n;
     }
 
+    // Buffers that belong to a capture's graph.
+    size_t captured_count() {
+        std::lock_guard<std::mutex> lk(mu_);
+        size_t n = 0;
+        for (auto& b : bufs_) n += b->capture != 0 && b->capture != kNoGraph && !b->returned ? 1 : 0;
+        return n;
+    }
+
     size_t held_count() {
         std::lock_guard<std::mutex> lk(mu_);
         size_t n = 0;
@@ -130,16 +183,22 @@ public:
     }
 
 private:
+    static constexpr size_t kCapturedGrain = size_t(2) << 20;
+    static constexpr uint64_t kNoGraph = ~uint64_t(0);
+
+    // Whether nothing can use a buffer once the device has drained.
+    static bool idle(const Buffer& b) { return !b.held && (b.capture == 0 || b.returned); }
+
     // Frees the idle buffers `which` selects, after the device has drained.
     template <class Pred>
     void retire_idle_locked(Pred which) {
         bool any = false;
-        for (auto& b : bufs_) any = any || (!b->held && which(*b));
+        for (auto& b : bufs_) any = any || (idle(*b) && which(*b));
         if (!any) return;
         b_.sync_device();
         for (size_t i = 0; i < bufs_.size();) {
             Buffer* b = bufs_[i].get();
-            if (b->held || !which(*b)) {
+            if (!idle(*b) || !which(*b)) {
                 ++i;
                 continue;
             }

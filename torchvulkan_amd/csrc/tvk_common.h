@@ -36,8 +36,9 @@ hipStream_t device_stream(int device);
 // current device. The lease ends when the object is destroyed, after the
 // call's launches. A buffer is only ever leased again for the same stream, so
 // stream order puts this call's kernels before the next holder's; buffers are
-// freed only after the device has drained, never while a lease holds them
-// (scratch_pool.h).
+// freed only after the device has drained, never while a lease holds them. A
+// captured call gets memory that stays the graph's until the graph and all its
+// executables are gone (scratch_pool.h).
 class Scratch {
 public:
     Scratch() = default;
@@ -48,22 +49,17 @@ public:
     // on `stream`; NULL when it cannot be allocated. One lease per object: a
     // second call ends the first lease.
     void* get(size_t bytes, hipStream_t stream);
-    // The same from a buffer that the stream's earlier calls have left idle,
-    // NULL without one: allocates nothing, so a captured call may ask.
-    void* get_idle(size_t bytes, hipStream_t stream);
     void release();
 
 private:
-    void* lease(size_t bytes, hipStream_t stream, bool idle_only);
     void* lease_ = nullptr;
     int device_ = -1;
     hipStream_t stream_ = nullptr;
 };
 
 // Whether a call that can do without may lease scratch for kernels on
-// `stream`: not while the stream is captured (a graph may be replayed on
-// another stream, where the pool's ownership by stream does not hold, and
-// capture must not allocate), nor on hipStreamPerThread, a handle that stands
+// `stream`: not while the stream is captured (the graph would keep the memory
+// for as long as it lives), nor on hipStreamPerThread, a handle that stands
 // for a stream of each thread.
 bool scratch_usable(hipStream_t stream);
 
