@@ -1,5 +1,6 @@
-"""Kernel families of grad weights whose channels-last copies would not fit
-the ring kernel's 2 GiB buffers (no GPU: the descriptors are not run)."""
+"""Kernel families of grad weights of odd planes: where the ring kernel's
+channels-last copies would not fit its 2 GiB buffers, and where there are too
+few output pixels for it (no GPU: the descriptors are not run)."""
 from __future__ import annotations
 
 import pytest
@@ -16,3 +17,17 @@ def test_bordered_copy_past_2_gib(batch, ring):
     assert (batch * 512 * 9 * 9 * 2 < 2**31) == ring and batch * 512 * 49 < 2**30
     names = _abi.conv_candidates(d, _abi.TVK_CONV_WGRAD)
     assert names == ["conv_ring", "conv_implicit_gemm"] if ring else names == ["conv_implicit_gemm"]
+
+
+# output pixels at and below its lines of 192 (up to 128 output channels) and 512
+@pytest.mark.parametrize("batch,hw,kernel,stride,cin,cout,ring", [
+    (1, 14, 3, 1, 64, 128, True), (3, 14, 3, 2, 64, 128, False), (1, 7, 3, 1, 512, 512, False), (1, 7, 1, 1, 8, 64, False),
+    (12, 7, 3, 2, 64, 64, True), (11, 7, 3, 2, 64, 64, False),      # 192 and 176 pixels
+    (1, 14, 3, 1, 64, 136, False), (2, 14, 3, 1, 256, 256, False),
+    (32, 7, 3, 2, 256, 256, True), (31, 7, 3, 2, 256, 256, False),   # 512 and 496 pixels
+])
+def test_few_output_pixels(batch, hw, kernel, stride, cin, cout, ring):
+    d = _abi.make_convnd_desc((batch, cin, hw, hw), (cout, cin, kernel, kernel), torch.float16, stride=stride,
+                              padding=kernel // 2)
+    d.x = d.weight = d.y = 256
+    assert ("conv_ring" in _abi.conv_candidates(d, _abi.TVK_CONV_WGRAD)) == ring

@@ -2116,8 +2116,12 @@ bool conv_ring_applies(const tvk_conv_desc& d, int mode) {
     if (!al16(d.x) || !al16(d.weight) || !al16(d.y)) return false;
     if (mode == 1 && (d.stride[0] > 4 || d.stride[1] > 4)) return false;
     // planes of other than whole 32-pixel stages read dy channels-last, in 8-channel chunks; the generic kernel takes
-    // the ones whose bordered copy would pass 2 GiB
-    if (conv_ring_dy_last(d, mode) && (d.c_out % 8 != 0 || wgrad_bordered_bytes(d, wgrad_border(d)) >= (int64_t(1) << 31)))
+    // the ones whose bordered copy would pass 2 GiB, and few output pixels: below 512 K is not split, and a tile's
+    // direct stores to dW, 2 bytes a row of taps apart, outlast the products they follow (bfloat16 64 -> 64, 3x3: 49
+    // pixels 9.8 us generic, 17.5 here; 196: 22.4 and 20.4; 512 -> 512: 196 pixels 30.5 and 48.5, 392: 50.8 and 53.5,
+    // 512: 230 and 54)
+    if (conv_ring_dy_last(d, mode) && (d.c_out % 8 != 0 || wgrad_bordered_bytes(d, wgrad_border(d)) >= (int64_t(1) << 31) ||
+                                       d.n * d.h_out * d.w_out < (d.c_out > 128 ? 512 : 192)))
         return false;
     // 32-bit element offsets inside the kernels
     const int64_t big = std::max({d.n * d.c_in * d.h * d.w, d.n * d.c_out * d.h_out * d.w_out, d.c_out * d.c_in * d.kh * d.kw});
