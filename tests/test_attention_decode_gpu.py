@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from oracle import oracle as orc
+from tests.kernel_names import kernels
 from tests.test_attention_gpu import DEV, assert_close, check, f64, rand
 from torchvulkan_amd import _abi
 
@@ -127,3 +128,26 @@ def test_non_finite_values(gpu, batch, heads, new, keys, dim):
     ro, rl = orc.attention(f64(q), f64(k), f64(torch.nan_to_num(v, 0.0, 0.0, 0.0)), None, False)
     assert_close(out[..., finite], ro[..., finite], dtype, "finite columns")
     assert np.allclose(f64(lse), rl, rtol=1e-3, atol=1e-3)
+
+
+# batch, (heads), queries, keys, dim, mask, packed: both sides of the lines between this kernel and the tiled forward
+@pytest.mark.parametrize("batch,heads,new,keys,dim,mask,packed", [
+    (1, (8, 8), 16, 64, 128, False, False), (1, (8, 8), 16, 65, 128, False, True),       # a head's own keys: one tile
+    (2, (16, 4), 4, 33, 128, False, True), (2, (16, 4), 5, 33, 128, False, False),       # 16 and 20 rows
+    (1, (16, 4), 16, 512, 128, False, False), (1, (16, 4), 16, 513, 128, False, True),
+    (1, (16, 4), 5, 448, 128, False, False), (1, (16, 4), 5, 449, 128, False, True),
+    (2, (32, 1), 1, 384, 64, False, False), (2, (32, 1), 1, 385, 64, False, True),
+    (2, (32, 1), 1, 384, 80, False, False), (2, (32, 1), 1, 385, 96, False, True),
+    (8, (32, 8), 5, 300, 128, False, False), (9, (32, 8), 5, 300, 128, False, True),   # a round of heads
+    (16, (32, 8), 5, 64, 128, False, False), (17, (32, 8), 5, 64, 128, False, True),
+    (32, (32, 8), 16, 64, 64, False, False), (33, (32, 8), 16, 64, 64, False, True),
+    (8, (32, 8), 16, 64, 128, True, False), (8, (32, 8), 16, 65, 128, True, True), (9, (32, 8), 16, 64, 64, True, True),
+])
+def test_dispatch(gpu, batch, heads, new, keys, dim, mask, packed):
+    dtype = torch.float16
+    q, k, v = (rand((batch, h, n, dim), dtype, i) for i, (h, n) in enumerate(((heads[0], new), (heads[1], keys), (heads[1], keys))))
+    bias = rand((batch, 1, 1, keys), dtype, 4) if mask else None
+    qd, kd, vd, bd = (None if t is None else t.to(DEV) for t in (q, k, v, bias))
+    names = kernels(lambda: _abi.attention_fwd(qd, kd, vd, bd))
+    assert any("attn_decode_kernel" in n for n in names) == packed and any("attn_fwd" in n for n in names) != packed, names
+    check(q[:1], k[:1], v[:1], bias=None if bias is None else bias[:1], what="first batch")

@@ -67,7 +67,7 @@ tvk_status fused_fwd(const tvk_attention_desc* d) {
                 d->out_stride[1] % 4 == 0 && d->out_stride[0] % 4 == 0;
     const hipStream_t s = resolve_stream(d->stream);
     const bool bias = d->bias != nullptr;
-    if (attn_decode_applies(a, causal, d->batch, d->heads_q)) {
+    if (attn_decode_applies(a, causal, bias, d->batch, d->heads_q)) {
         attn_decode_fwd(d->dtype, a, bias, d->batch, d->heads_q, s);
     } else if (d->head_dim != 64 && d->head_dim != 128) {
         if (!attn_part_fwd(d->dtype, a, causal, bias, d->batch, d->heads_q, d->len_q, s))

@@ -416,17 +416,31 @@ void launch(const DecodeArgs& p, bool bias, int ct, dim3 grid, int64_t all_rows,
 // for 256, 30.9 for 768), as long as every wave keeps a tile (32/8 heads x
 // 1000 x 64: 6.1 us, 6.5 with two tiles a wave) and into at most 32 parts: the
 // last workgroup reads them one after another (1 x 32/8 x 16000 x 128: 17.7 us
-// in 32 parts, 21.3 in 63).
-constexpr int kTargetGroups = 512, kMaxSplits = 32;
+// in 32 parts, 21.3 in 63). Two column blocks merge twice the rows: below 16
+// tiles one part (64 x 8/2 heads, 5 queries x 256 x 128: 8.9 us, 12.2 in two; 512
+// keys 14.2, 12.1 in four), except with a bias, whose loads the parts share out.
+constexpr int kTargetGroups = 512, kMaxSplits = 32, kMinTiles2 = 16;
 
 }  // namespace
 
-bool attn_decode_applies(const AttnArgs& a, bool causal, int64_t batch, int64_t heads) {
+bool attn_decode_applies(const AttnArgs& a, bool causal, bool bias, int64_t batch, int64_t heads) {
     // row offsets inside a tile are 32-bit
     const auto row_ok = [](int64_t st) { return (DC_BN * st + 128) * 2 < (int64_t)0x7fffffff; };
     // one tile of keys and no head to share them with leaves nothing to split or pack: the tiled forward is as fast
     // (64 x 8 heads x 64 keys of 64, 16 queries: 4.2 us there, 4.5 here; 128 keys: 7.0 there, 6.4 here)
     if (a.group == 1 && a.S <= AT_BN) return false;
+    // More than 16 query rows a key/value head are two column blocks a wave: over short sequences, where the tiled
+    // forward's workgroup a query head is at most two rounds, the blocks' merge costs more than the shared keys save.
+    // Tiled and here, float16 4 x 8/2 heads, 16 queries: of 128, 65 keys 5.7 and 6.9 us, 256 keys 7.6 and 12.4, 512 keys
+    // 12.1 and 12.8, 700 keys 16.0 and 14.1; of 64, 128 keys 4.4 and 5.2, 400 keys 8.7 and 8.9 (7.7 in one part), 700
+    // keys 12.1 and 9.0. With 1024 heads (64 x 16/1) of 64: 64 keys 5.1 and 6.4, 65 keys 7.3 and 6.4. With a bias, whose
+    // values the tiled forward loads a head at a time, only a single tile of keys (4 x 64/8 heads, 5 queries, of 128: 64
+    // keys 6.7 and 8.2, 65 keys 8.7 and 8.3).
+    if (a.L * a.group > 16) {
+        const int64_t bh = batch * heads;
+        if (a.S <= AT_BN && bh <= (bias ? 256 : a.hd <= 64 ? 1024 : 512)) return false;
+        if (!bias && a.S <= (a.hd <= 96 ? 6 : a.L * a.group <= 32 ? 7 : 8) * AT_BN && bh <= 256) return false;
+    }
     return !causal && a.L <= 16 && a.S > 0 && row_ok(a.sk[2]) && row_ok(a.sv[2]) &&
            batch * (heads / a.group) * (((int64_t)a.L * a.group + 15) / 16) <= (int64_t)0x7fffffff;
 }
@@ -440,7 +454,8 @@ void attn_decode_fwd(int dtype, const AttnArgs& args, bool bias, int64_t batch, 
     p.nrb = (p.rows + 16 * ct - 1) / (16 * ct);
     const int64_t bhk = batch * p.kvh, base = bhk * p.nrb, all_rows = bhk * p.rows;
     const int tiles = (args.S + DC_BN - 1) / DC_BN;
-    const int want = (int)std::min<int64_t>(std::max<int64_t>(1, kTargetGroups / base), std::max(1, std::min(kMaxSplits, tiles / DC_WAVES)));
+    const int most = ct == 2 && !bias && tiles < kMinTiles2 ? 1 : std::max(1, std::min(kMaxSplits, tiles / DC_WAVES));
+    const int want = (int)std::min<int64_t>(std::max<int64_t>(1, kTargetGroups / base), most);
     p.per = ((tiles + want - 1) / want + DC_WAVES - 1) / DC_WAVES * DC_WAVES;
     p.splits = (tiles + p.per - 1) / p.per;
     Scratch scratch;

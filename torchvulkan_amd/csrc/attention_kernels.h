@@ -1250,7 +1250,7 @@ bool attn_part_bwd(int dtype, const AttnBwdArgs& a, bool causal, bool bias, int6
                    hipStream_t s);
 
 // Few queries over many keys (attention_decode.hip): L <= 16, no causal mask.
-bool attn_decode_applies(const AttnArgs& a, bool causal, int64_t batch, int64_t heads);
+bool attn_decode_applies(const AttnArgs& a, bool causal, bool bias, int64_t batch, int64_t heads);
 void attn_decode_fwd(int dtype, const AttnArgs& a, bool bias, int64_t batch, int64_t heads, hipStream_t s);
 
 }  // namespace tvk
