@@ -101,3 +101,64 @@ def test_wide_kernel(gpu, dim, batch, heads, lens, causal):
         assert_close(f64(out[b:b + 1, h:h + 1]), ro, dtype, f"b {b} h {h}")
         assert (abs(f64(lse[b:b + 1, h:h + 1]) - rl) <= 1e-3 * (abs(rl) + 1)).all()
     assert not out.isnan().any()
+
+
+# the same kernel over several query blocks and key tiles (a tile's buffer is loaded again from the third on), heads
+# and batches at both ends and in the middle; the last lengths have fewer queries than keys
+@pytest.mark.parametrize("dim,batch,heads", [(128, 16, 32), (104, 16, 32), (80, 16, 32), (64, 16, 32)])
+@pytest.mark.parametrize("lens,causal", [((300, 300), True), ((300, 300), False), ((200, 391), False), ((257, 449), True)])
+def test_wide_kernel_over_many_tiles(gpu, dim, batch, heads, lens, causal):
+    from tests.kernel_names import kernels
+    from torchvulkan_amd import _abi
+
+    dtype = torch.bfloat16 if dim % 16 else torch.float16
+    n, s = lens
+    q = rand((batch, n, heads, dim), dtype, 1).to(DEV).transpose(1, 2)
+    k, v = (rand((batch, s, 2, dim), dtype, i).to(DEV).transpose(1, 2) for i in (2, 3))
+    got = []
+    names = kernels(lambda: got.append(_abi.attention_fwd(q, k, v, None, causal)))
+    assert [x for x in names if "attn_fwd_wide_kernel" in x] == names and names, names
+    out, lse = got[0]
+    for b, h in ((0, 0), (batch // 2, heads // 2), (batch - 1, heads - 1)):
+        hk = h // (heads // 2)
+        ro, rl = orc.attention(f64(q[b:b + 1, h:h + 1]), f64(k[b:b + 1, hk:hk + 1]), f64(v[b:b + 1, hk:hk + 1]), None, causal)
+        assert_close(f64(out[b:b + 1, h:h + 1]), ro, dtype, f"b {b} h {h}")
+        assert (abs(f64(lse[b:b + 1, h:h + 1]) - rl) <= 1e-3 * (abs(rl) + 1)).all()
+
+
+# heads, queries, dim, wide: both sides of the rule between the two forwards
+@pytest.mark.parametrize("batch,heads,n,dim,wide", [
+    (16, 32, 64, 128, False), (16, 32, 65, 128, True), (64, 32, 64, 104, False),
+    (7, 73, 128, 96, False), (16, 16, 129, 80, True),      # 511 and 512 workgroups of 128 queries
+    (32, 32, 64, 64, False), (32, 32, 65, 64, True), (64, 32, 17, 64, True), (89, 23, 17, 64, False),
+    (16, 32, 192, 64, False), (16, 32, 193, 64, True), (16, 32, 192, 40, False), (16, 32, 193, 40, True),
+])
+def test_wide_dispatch(gpu, batch, heads, n, dim, wide):
+    from tests.kernel_names import kernels
+    from torchvulkan_amd import _abi
+
+    q = torch.ones((batch, heads, n, dim), dtype=torch.float16, device=DEV)
+    names = kernels(lambda: _abi.attention_fwd(q, q, q, None, True))
+    assert all(("wide" in x) == wide for x in names) and names, names
+
+
+def test_two_query_columns_with_a_bias(gpu):
+    # head dim 64 with a bias on 2048 workgroups of 128 queries: the 64-query kernel's two-column form
+    from tests.kernel_names import kernels
+    from torchvulkan_amd import _abi
+
+    dtype, batch, heads, n, s = torch.float16, 32, 32, 200, 130
+    q, k, v = rand((batch, heads, n, 64), dtype, 1), rand((batch, 4, s, 64), dtype, 2), rand((batch, 4, s, 64), dtype, 3)
+    bias = rand((1, heads, 1, s), dtype, 4)
+    bias[..., 100:] = float("-inf")
+    for causal in (False, True):
+        got = []
+        qd, kd, vd, bd = (t.to(DEV) for t in (q, k, v, bias))
+        names = kernels(lambda: got.append(_abi.attention_fwd(qd, kd, vd, bd, causal)))
+        assert len(names) == 1 and "attn_fwd_kernel" in names[0], names
+        for b, h in ((0, 0), (13, 17), (31, 31)):
+            hk = h // 8
+            ro, rl = orc.attention(f64(q[b:b + 1, h:h + 1]), f64(k[b:b + 1, hk:hk + 1]), f64(v[b:b + 1, hk:hk + 1]),
+                                   f64(bias[:, h:h + 1].expand(1, 1, n, s)), causal)
+            assert_close(f64(got[0][0][b:b + 1, h:h + 1]), ro, dtype, f"b {b} h {h} causal {causal}")
+            assert (abs(f64(got[0][1][b:b + 1, h:h + 1]) - rl) <= 1e-3 * (abs(rl) + 1)).all()

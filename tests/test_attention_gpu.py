@@ -64,8 +64,8 @@ def test_ragged_lengths_and_head_dim_128(gpu, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [False, True])
 def test_wide_grid_two_query_columns_per_wave(gpu, dtype, causal):
-    # batch*heads*ceil(L/128) >= 2048 selects 128-query workgroups (two 16-query
-    # columns per wave); the oracle checks a few (batch, head) slices
+    # a grid of 128-query workgroups (two 16-query columns per wave, the wide
+    # kernel without a bias); the oracle checks a few (batch, head) slices
     B, Hq, Hk, L, D = 16, 16, 4, 1024, 64
     q, k, v = rand((B, Hq, L, D), dtype, 60), rand((B, Hk, L, D), dtype, 61), rand((B, Hk, L, D), dtype, 62)
     out, lse = _abi.attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV), None, causal)

@@ -693,17 +693,22 @@ void launch_attn_q(AttnArgs a, bool causal, bool bias, int64_t bh, int64_t L, hi
 }
 
 // Two query columns a wave (the wide kernel) where its 128-query workgroups
-// still fill the device: from two a CU (head_dim 128, 8 heads x 4608: 288 of
-// them, 94 us on the 64-query kernel, 138 wide; 512 of them, 22.2 against 17.0),
-// at head_dim 64, where less LDS lets more of the 64-query workgroups share a
-// CU, from four (512 of 32 x 8 x 256: 10.76 against 10.86; 1024 of 16 x 16 x
-// 512: 35.2 against 31.3). With a bias the 64-query kernel, at head_dim 64 on
-// large grids in its two-column form.
+// still fill the device: above head_dim 64 from two a CU (head_dim 128, 8 heads
+// x 4608: 288 of them, 94 us on the 64-query kernel, 138 wide; 512 of them,
+// 22.2 against 17.0) of more than 64 queries (its second half of a workgroup
+// idle: 4096 heads x 64, 49 us against 61); at head_dim 64, where less LDS lets
+// more of the 64-query workgroups share a CU, from eight of those a CU (1536 of
+// 512 heads x 192: 12.3 against 13.2; 2048 of 512 x 256: 17.0 against 15.7; 1024
+// of 1024 x 64: 6.9 against 8.9; 2048 of 2048 x 64: 15.0 against 14.0). With a
+// bias the 64-query kernel, at head_dim 64 on large grids in its two-column
+// form.
 template <int DT, int D, bool PART>
 void launch_attn(const AttnArgs& a, bool causal, bool bias, int64_t batch, int64_t heads, int64_t L, hipStream_t s) {
     if constexpr (D >= 64) {
         const bool rows_ok = (AT_BN * a.sk[2] + 128) * 2 < (int64_t)0x7fffffff && (AT_BN * a.sv[2] + 128) * 2 < (int64_t)0x7fffffff;
-        if (!bias && rows_ok && batch * heads * ((L + 127) / 128) >= (D == 64 ? 1024 : 512)) {
+        const int64_t bh = batch * heads;
+        const bool full = D == 64 ? bh * ((L + 63) / 64) >= 2048 : L > 64 && bh * ((L + 127) / 128) >= 512;
+        if (!bias && rows_ok && full) {
             AttnArgs w = a;
             w.nqb = (int)((L + 127) / 128);
             w.BH = (int)(batch * heads);
