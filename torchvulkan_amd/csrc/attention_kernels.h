@@ -683,7 +683,10 @@ void launch_attn_q(AttnArgs a, bool causal, bool bias, int64_t bh, int64_t L, hi
     a.nqb = (int)((L + BMQ - 1) / BMQ);
     a.BH = (int)bh;
     const dim3 grid((unsigned)(a.nqb * bh)), block(64 * AT_WAVES);
-    if (causal) {
+    if constexpr (QPW == 2) {   // (without a bias: the wide kernel)
+        if (causal) hipLaunchKernelGGL((attn_fwd_kernel<DT, D, true, true, QPW, PART>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((attn_fwd_kernel<DT, D, false, true, QPW, PART>), grid, block, 0, s, a);
+    } else if (causal) {
         if (bias) hipLaunchKernelGGL((attn_fwd_kernel<DT, D, true, true, QPW, PART>), grid, block, 0, s, a);
         else hipLaunchKernelGGL((attn_fwd_kernel<DT, D, true, false, QPW, PART>), grid, block, 0, s, a);
     } else {
@@ -719,7 +722,7 @@ void launch_attn(const AttnArgs& a, bool causal, bool bias, int64_t batch, int64
         }
     }
     if constexpr (D == 64 && !PART) {
-        if (batch * heads * ((L + 127) / 128) >= 2048) {
+        if (bias && batch * heads * ((L + 127) / 128) >= 2048) {
             launch_attn_q<DT, D, 2, PART>(a, causal, bias, batch * heads, L, s);
             return;
         }

@@ -406,18 +406,19 @@ __global__ __launch_bounds__(64 * ring_waves(BM, BN)) void conv_ring_kernel(Conv
 // launch: w[co][c][t] -> wout[co][t][c] (forward) or wout[c][t][co] (grad
 // input). Column block nx - 1, when the plane has a border, zeroes the border
 // pixels of its channels (the rows above and below, then the columns left and
-// right of each image row); the others copy 64 channels x PX pixels.
-// VEC (C % 8 == 0): PX = 256, no LDS. A lane loads 8 pixels of 8 channels
-// (eight 16-byte loads; 8 lanes read 128 contiguous bytes of a channel row),
-// transposes the 8x8 block of 16-bit elements in registers and stores 8 pixels
-// of 8 channels (8 lanes write 128 contiguous bytes of a pixel). The loads
+// right of each image row); the others copy 64 channels x 256 pixels. Channels
+// come in whole eights (conv_ring_applies), so no LDS: a lane loads 8 pixels of
+// 8 channels (eight 16-byte loads; 8 lanes read 128 contiguous bytes of a
+// channel row), transposes the 8x8 block of 16-bit elements in registers and
+// stores 8 pixels of 8 channels (8 lanes write 128 contiguous bytes of a pixel). The loads
 // need no alignment beyond the element's, so any plane takes this path (14 x
 // 14 and 7 x 7 planes went through LDS one element at a time: 12-15 us for
 // 32 x 256 x 14 x 14 and its weight, 8-9 here); the last chunk of a plane whose
 // pixels are no multiple of 8 goes element by element.
-// Otherwise PX = 64 through an LDS tile, element accesses.
 // A grad weight's launch copies two tensors: workgroups past the first
 // tensor's take the second's.
+constexpr int NHWC_PX = 256;   // pixels of a workgroup
+
 struct WeightPermute {
     const uint16_t* w = nullptr;
     uint16_t* out = nullptr;
@@ -447,7 +448,7 @@ __device__ inline void permute_weight(const WeightPermute& wp, int blk, int nb) 
     }
 }
 
-__device__ inline void zero_border(const NhwcArgs& a, uint16_t* d, int c0, bool vec) {
+__device__ inline void zero_border(const NhwcArgs& a, uint16_t* d, int c0) {
     const int rows = a.Hs - a.H, cols = a.Ws - a.W;   // border rows (whole width), border columns per image row
     const int npix = rows * a.Ws + a.H * cols;
     for (int e = threadIdx.x; e < npix * 8; e += 256) {
@@ -464,9 +465,7 @@ __device__ inline void zero_border(const NhwcArgs& a, uint16_t* d, int c0, bool 
             wq = k < a.pl ? k : k + a.W;
         }
         uint16_t* o = d + ((int64_t)hp * a.Ws + wq) * a.C + c;
-        if (vec && c + 8 <= a.C) *reinterpret_cast<u32x4*>(o) = u32x4{0, 0, 0, 0};
-        else
-            for (int k = 0; k < 8 && c + k < a.C; ++k) o[k] = 0;
+        *reinterpret_cast<u32x4*>(o) = u32x4{0, 0, 0, 0};
     }
 }
 
@@ -477,7 +476,6 @@ __device__ inline u32x4 load16_any(const uint16_t* p) {
     return v;
 }
 
-template <bool VEC>
 __global__ __launch_bounds__(256) void nchw_to_nhwc_kernel(NhwcSet set) {
     int b = blockIdx.x;
     const int copies = set.t[0].copy_blocks + set.t[1].copy_blocks;
@@ -491,66 +489,43 @@ __global__ __launch_bounds__(256) void nchw_to_nhwc_kernel(NhwcSet set) {
     const int C = a.C, W = a.W, HW = a.H * a.W;
     uint16_t* d = a.dst + (int64_t)img * a.Hs * a.Ws * C;
     if (bx >= a.nblk) {
-        zero_border(a, d, c0, VEC);
+        zero_border(a, d, c0);
         return;
     }
     const uint16_t* s = a.src + (int64_t)img * C * HW;
-    if constexpr (VEC) {
-        const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-        const int c = c0 + (lane % 8) * 8;
-        const int px = bx * 256 + wave * 64 + (lane / 8) * 8;
-        if (c >= C || px >= HW) return;
-        u32x4 r[8];
-        if (px + 8 <= HW) {
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    const int c = c0 + (lane % 8) * 8;
+    const int px = bx * NHWC_PX + wave * 64 + (lane / 8) * 8;
+    if (c >= C || px >= HW) return;
+    u32x4 r[8];
+    if (px + 8 <= HW) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) r[i] = load16_any(s + (int64_t)(c + i) * HW + px);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint16_t* q = s + (int64_t)(c + i) * HW + px + 2 * e;
-                    const uint32_t lo = px + 2 * e < HW ? q[0] : 0, hi = px + 2 * e + 1 < HW ? q[1] : 0;
-                    r[i][e] = lo | (hi << 16);
-                }
-        }
-        int h = px / W, w = px - h * W;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (px + j >= HW) break;
-            // pixel px + j: channel pairs (2k, 2k + 1) packed low/high
-            uint32_t v[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint32_t lo = r[2 * k][j / 2], hi = r[2 * k + 1][j / 2];
-                v[k] = (j % 2 == 0) ? ((lo & 0xffffu) | (hi << 16)) : ((lo >> 16) | (hi & 0xffff0000u));
-            }
-            *reinterpret_cast<u32x4*>(d + ((int64_t)(h + a.pt) * a.Ws + w + a.pl) * C + c) = u32x4{v[0], v[1], v[2], v[3]};
-            if (++w == W) {
-                w = 0;
-                ++h;
-            }
-        }
+        for (int i = 0; i < 8; ++i) r[i] = load16_any(s + (int64_t)(c + i) * HW + px);
     } else {
-        __shared__ uint16_t tile[64][72];
-        const int p0 = bx * 64;
 #pragma unroll
-        for (int e = threadIdx.x; e < 64 * 8; e += 256) {
-            const int c = e / 8, q = (e % 8) * 8;
-            if (c0 + c >= C) continue;
-            for (int k = 0; k < 8; ++k)
-                if (p0 + q + k < HW) tile[c][q + k] = s[(int64_t)(c0 + c) * HW + p0 + q + k];
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint16_t* q = s + (int64_t)(c + i) * HW + px + 2 * e;
+                const uint32_t lo = px + 2 * e < HW ? q[0] : 0, hi = px + 2 * e + 1 < HW ? q[1] : 0;
+                r[i][e] = lo | (hi << 16);
+            }
+    }
+    int h = px / W, w = px - h * W;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        if (px + j >= HW) break;
+        // pixel px + j: channel pairs (2k, 2k + 1) packed low/high
+        uint32_t v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t lo = r[2 * k][j / 2], hi = r[2 * k + 1][j / 2];
+            v[k] = (j % 2 == 0) ? ((lo & 0xffffu) | (hi << 16)) : ((lo >> 16) | (hi & 0xffff0000u));
         }
-        __syncthreads();
-#pragma unroll
-        for (int e = threadIdx.x; e < 64 * 8; e += 256) {
-            const int q = e / 8, c = (e % 8) * 8;
-            const int px = p0 + q;
-            if (px >= HW) continue;
-            const int h = px / W, w = px - h * W;
-            uint16_t* o = d + ((int64_t)(h + a.pt) * a.Ws + w + a.pl) * C + c0 + c;
-            for (int k = 0; k < 8; ++k)
-                if (c0 + c + k < C) o[k] = tile[c + k][q];
+        *reinterpret_cast<u32x4*>(d + ((int64_t)(h + a.pt) * a.Ws + w + a.pl) * C + c) = u32x4{v[0], v[1], v[2], v[3]};
+        if (++w == W) {
+            w = 0;
+            ++h;
         }
     }
 }
@@ -641,9 +616,6 @@ struct NhwcCopy {
 void launch_nhwc(const NhwcCopy* copies, int count, int n, hipStream_t s, const WeightPermute& wp = WeightPermute()) {
     NhwcSet set;
     memset(&set.t, 0, sizeof(set.t));
-    bool vec = true;
-    for (int i = 0; i < count; ++i) vec = vec && copies[i].C % 8 == 0;
-    const int px = vec ? 256 : 64;
     int blocks = 0;
     for (int i = 0; i < count; ++i) {
         const NhwcCopy& q = copies[i];
@@ -653,7 +625,7 @@ void launch_nhwc(const NhwcCopy* copies, int count, int n, hipStream_t s, const 
         a.C = q.C; a.H = q.H; a.W = q.W;
         a.Hs = q.H + q.bd.pt + q.bd.pb; a.Ws = q.W + q.bd.pl + q.bd.pr;
         a.pt = q.bd.pt; a.pl = q.bd.pl;
-        a.nblk = (q.H * q.W + px - 1) / px;
+        a.nblk = (q.H * q.W + NHWC_PX - 1) / NHWC_PX;
         const bool border = a.Hs > q.H || a.Ws > q.W;
         a.nx = a.nblk + (border ? 1 : 0);
         a.cy = (q.C + 63) / 64;
@@ -664,8 +636,7 @@ void launch_nhwc(const NhwcCopy* copies, int count, int n, hipStream_t s, const 
     const int64_t wn = (int64_t)wp.cout * wp.cin * wp.taps;
     const int wblocks = wp.w ? (int)std::min<int64_t>((wn + 255) / 256, 1024) : 0;
     const dim3 grid((unsigned)(blocks + wblocks));
-    if (vec) hipLaunchKernelGGL(nchw_to_nhwc_kernel<true>, grid, dim3(256), 0, s, set);
-    else hipLaunchKernelGGL(nchw_to_nhwc_kernel<false>, grid, dim3(256), 0, s, set);
+    hipLaunchKernelGGL(nchw_to_nhwc_kernel, grid, dim3(256), 0, s, set);
 }
 
 // Border that keeps rows lo + i*step + [tap_lo, tap_hi] for i in [0, count)
