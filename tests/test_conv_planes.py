@@ -31,3 +31,12 @@ def test_few_output_pixels(batch, hw, kernel, stride, cin, cout, ring):
                               padding=kernel // 2)
     d.x = d.weight = d.y = 256
     assert ("conv_ring" in _abi.conv_candidates(d, _abi.TVK_CONV_WGRAD)) == ring
+
+
+# the copies' launch holds at most 2^24 workgroups (2^32 threads): batches of tiny planes past it
+@pytest.mark.parametrize("batch,hw,kernel,ring", [(1 << 20, 1, 1, True), (1 << 23, 1, 1, False), (1 << 25, 1, 1, False),
+                                                  ((1 << 22) - 1, 3, 3, True), (1 << 23, 3, 3, False)])
+def test_more_workgroups_than_a_launch_holds(batch, hw, kernel, ring):
+    d = _abi.make_convnd_desc((batch, 8, hw, hw), (8, 8, kernel, kernel), torch.float16, stride=1, padding=kernel // 2)
+    d.x = d.weight = d.y = 256
+    assert ("conv_ring" in _abi.conv_candidates(d, _abi.TVK_CONV_WGRAD)) == ring

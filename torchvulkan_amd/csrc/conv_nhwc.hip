@@ -655,6 +655,12 @@ Border wgrad_border(const tvk_conv_desc& d) {
     return bd;
 }
 
+// Workgroups of one tensor's layout copy.
+int64_t nhwc_blocks(int64_t n, int64_t c, int64_t h, int64_t w, const Border& bd) {
+    const bool border = bd.pt + bd.pb + bd.pl + bd.pr > 0;
+    return n * ((c + 63) / 64) * ((h * w + NHWC_PX - 1) / NHWC_PX + (border ? 1 : 0));
+}
+
 int64_t wgrad_bordered_bytes(const tvk_conv_desc& d, const Border& bd) {
     return d.n * d.c_in * (d.h + bd.pt + bd.pb) * (d.w + bd.pl + bd.pr) * 2;
 }
@@ -2087,11 +2093,13 @@ bool conv_ring_applies(const tvk_conv_desc& d, int mode) {
     if (!al16(d.x) || !al16(d.weight) || !al16(d.y)) return false;
     if (mode == 1 && (d.stride[0] > 4 || d.stride[1] > 4)) return false;
     // planes of other than whole 32-pixel stages read dy channels-last, in 8-channel chunks; the generic kernel takes
-    // the ones whose bordered copy would pass 2 GiB, and few output pixels: below 512 K is not split, and a tile's
+    // the ones whose bordered copy would pass 2 GiB or whose copies a launch's 2^32 threads, and few output pixels: below 512 K is not split, and a tile's
     // direct stores to dW, 2 bytes a row of taps apart, outlast the products they follow (bfloat16 64 -> 64, 3x3: 49
     // pixels 9.8 us generic, 17.5 here; 196: 22.4 and 20.4; 512 -> 512: 196 pixels 30.5 and 48.5, 392: 50.8 and 53.5,
     // 512: 230 and 54)
     if (conv_ring_dy_last(d, mode) && (d.c_out % 8 != 0 || wgrad_bordered_bytes(d, wgrad_border(d)) >= (int64_t(1) << 31) ||
+                                       nhwc_blocks(d.n, d.c_in, d.h, d.w, wgrad_border(d)) +
+                                               nhwc_blocks(d.n, d.c_out, d.h_out, d.w_out, Border()) >= (int64_t(1) << 24) ||
                                        d.n * d.h_out * d.w_out < (d.c_out > 128 ? 512 : 192)))
         return false;
     // 32-bit element offsets inside the kernels
