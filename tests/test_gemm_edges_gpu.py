@@ -64,6 +64,17 @@ def test_row_edges(gpu, layout, m, n, k):
     product(layout, m, n, k, torch.bfloat16, out_pad=3)
 
 
+# a row's last chunk of 1 to 7 elements, in each of the ring's epilogues (none, ReLU and a bias, a bias off 16-byte
+# rows), between guard columns
+@pytest.mark.parametrize("n", range(1545, 1552))
+def test_row_tails(gpu, n):
+    plan = product("nn", 1500, n, 1032, torch.float16, out_pad=1)
+    product("tn", 1504, n, 72, torch.bfloat16, out_pad=2)
+    product("nn", 1500, n, 1032, torch.bfloat16, bias=True, out_pad=5)
+    product("nn", 1500, n, 1024, torch.float16, bias=True, act=_abi.TVK_ACT_RELU, out_pad=3)
+    assert plan == "gemm16_mfma_128x128"
+
+
 # split K with a masked end in the last chunk; N no multiple of 4 (padded rows of partials)
 @pytest.mark.parametrize("layout", ["nn", "tn", "nt"])
 @pytest.mark.parametrize("n", [640, 637])

@@ -467,12 +467,9 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                     h[e] = __builtin_bit_cast(uint16_t, elem<DT>::from_f32(v));
                 }
                 T* cp = Cb + (int64_t)row * p.sc[1] + col;
-                if (col + 8 <= p.N) {
-                    st_nt(reinterpret_cast<u32x4u*>(cp), u32x4u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
-                                                          (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)});
-                } else {
-                    for (int e = 0; e < 8 && col + e < p.N; ++e) cp[e] = __builtin_bit_cast(T, h[e]);
-                }
+                store_row8(reinterpret_cast<uint16_t*>(cp), u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
+                                                                  (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)},
+                           p.N - col);
             }
             __syncthreads();
         }
@@ -538,12 +535,9 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                     h[e] = __builtin_bit_cast(uint16_t, elem<DT>::from_f32(v));
                 }
                 T* cp = Cb + (int64_t)row * p.sc[1] + col;
-                if (full) {
-                    st_nt(reinterpret_cast<u32x4u*>(cp), u32x4u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
-                                                          (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)});
-                } else {
-                    for (int e = 0; e < 8 && col + e < p.N; ++e) cp[e] = __builtin_bit_cast(T, h[e]);
-                }
+                store_row8(reinterpret_cast<uint16_t*>(cp), u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
+                                                                  (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)},
+                           p.N - col);
             }
             __syncthreads();
         }
@@ -591,9 +585,10 @@ __global__ __launch_bounds__(dma_threads(BM, BN)) void gemm16_dma_kernel(GemmArg
                 h[e] = __builtin_bit_cast(uint16_t, elem<DT>::from_f32(v));
             }
             T* cp = Cb + (int64_t)row * p.sc[1] + (int64_t)col * p.sc[2];
-            if (vec_c && full) {
-                st_nt(reinterpret_cast<u32x4u*>(cp), u32x4u{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
-                                                      (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)});
+            if (vec_c) {
+                store_row8(reinterpret_cast<uint16_t*>(cp), u32x4{(uint32_t)h[0] | ((uint32_t)h[1] << 16), (uint32_t)h[2] | ((uint32_t)h[3] << 16),
+                                                                  (uint32_t)h[4] | ((uint32_t)h[5] << 16), (uint32_t)h[6] | ((uint32_t)h[7] << 16)},
+                           p.N - col);
             } else {
                 for (int e = 0; e < 8 && col + e < p.N; ++e) cp[(int64_t)e * p.sc[2]] = __builtin_bit_cast(T, h[e]);
             }
