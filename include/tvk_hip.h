@@ -527,9 +527,16 @@ tvk_status tvk_gemm(const tvk_gemm_desc* desc);
  * one stream do not. Results are those of tvk_gemm with the same kernel. */
 tvk_status tvk_gemm_noalloc(const tvk_gemm_desc* desc);
 
-/* Name of the kernel tvk_gemm would launch for `desc` (no launch). Used by
- * tests and the benchmark to state which path ran; replaces the tuner's
- * choice record (src/vulkan/autotuner.cpp:56-84). */
+/* Name of the plan tvk_gemm would run for `desc` (no launch): the kernel and
+ * its tile. Used by tests and the benchmark to state which path ran; replaces
+ * the tuner's choice record (src/vulkan/autotuner.cpp:56-84). Two names stand
+ * for more than one kernel, as the names that tuning files hold:
+ * "gemm16_mfma_256x256_w8" and "gemm16_mfma_128x128[_splitk]" run the LDS-ring
+ * kernel, on 256x256, 128x256 or 128x128 tiles by the product's size, where its
+ * operands need only masks past K (K a multiple of 8, off the 32 grid) or rows
+ * repacked to whole 16-byte chunks, and the register-staged kernel elsewhere;
+ * "gemm16_skinny_bk" is the family of few rows with a k-contiguous B, on its
+ * ring or the register kernel, K split or not. */
 tvk_status tvk_gemm_plan(const tvk_gemm_desc* desc, char* name, size_t name_len);
 
 /* ---- kernel-choice table ----------------------------------------------------

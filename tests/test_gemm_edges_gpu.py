@@ -8,6 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
+from tests.kernel_names import kernels
 from torchvulkan_amd import _abi
 
 pytestmark = pytest.mark.gpu
@@ -58,9 +59,9 @@ def test_k_edges(gpu, layout, k):
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn"])
 @pytest.mark.parametrize("m,n,k", [(1501, 1537, 1024), (1537, 1499, 1000), (1300, 2001, 93)])
 def test_row_edges(gpu, layout, m, n, k):
-    for bias, act in ((False, _abi.TVK_ACT_NONE), (True, _abi.TVK_ACT_RELU), (True, _abi.TVK_ACT_GELU)):
-        if act != _abi.TVK_ACT_GELU:   # (GELU's values are not exact: covered by the GEMM tests)
-            product(layout, m, n, k, torch.float16, bias=bias, act=act)
+    # (GELU's values are not exact: covered by the GEMM tests)
+    for bias, act in ((False, _abi.TVK_ACT_NONE), (True, _abi.TVK_ACT_RELU)):
+        product(layout, m, n, k, torch.float16, bias=bias, act=act)
     product(layout, m, n, k, torch.bfloat16, out_pad=3)
 
 
@@ -106,3 +107,27 @@ def test_batches(gpu):
     _abi.gemm(a.to(DEV).view(2, 3, 700, 104), b.to(DEV).view(2, 3, 104, 1003), c4)
     torch.cuda.synchronize()
     assert torch.equal(c.cpu().double(), want) and torch.equal(c4.cpu().double().view(6, 700, 1003), want)
+
+
+# which kernel runs under the plan's name: the ring (and its tile) or the register-staged kernel, on both sides of the
+# lines. m, n, k, batch, layout, ring tile
+@pytest.mark.parametrize("m,n,k,batch,layout,tile", [
+    (1500, 1544, 1040, 1, "nn", "128, 128"), (1500, 1544, 40, 1, "nn", "128, 128"), (1500, 1544, 24, 1, "nn", None),
+    (1501, 1537, 1024, 1, "nn", "128, 128"), (1501, 1537, 1024, 1, "tn", "128, 128"),
+    (1500, 1544, 1016, 1, "nt", None), (1500, 1544, 1032, 1, "nt", "128, 128"),   # two k-contiguous operands: from 1024
+    (2048, 2048, 1032, 1, "nt", "128, 128"), (2049, 2048, 1032, 1, "nt", None),   # to 256 tiles
+    (1280, 2064, 1032, 3, "nt", None), (3000, 3000, 1032, 1, "nt", "256, 256"), (4352, 104, 1032, 16, "nt", None),
+    (500, 640, 2056, 1, "nn", "128, 128"), (500, 640, 2056, 1, "nt", None),       # split K
+    (4096, 3008, 72, 1, "nt", "256, 256"), (4600, 4600, 104, 1, "nn", "128, 256"),
+])
+def test_kernel_of_a_plan(gpu, m, n, k, batch, layout, tile):
+    dtype = torch.float16
+    sh = (batch,) if batch > 1 else ()
+    a = torch.ones((*sh, k, m), dtype=dtype, device=DEV).transpose(-1, -2) if layout == "tn" else torch.ones((*sh, m, k), dtype=dtype, device=DEV)
+    b = torch.ones((*sh, n, k), dtype=dtype, device=DEV).transpose(-1, -2) if layout == "nt" else torch.ones((*sh, k, n), dtype=dtype, device=DEV)
+    c = torch.empty((*sh, m, n), dtype=dtype, device=DEV)
+    assert _abi.gemm_plan(a, b, c).startswith("gemm16_mfma_")
+    names = [x for x in kernels(lambda: _abi.gemm(a, b, c)) if "gemm16_" in x]
+    assert len(names) == 1 and ("gemm16_dma_kernel" in names[0]) == (tile is not None), names
+    assert tile is None or f", {tile}, 4, " in names[0], names
+    assert (c == k).all()

@@ -953,10 +953,17 @@ Plan make_plan(const tvk_gemm_desc& d) {
 //     x 904 24.4 -> 21.7. Two k-contiguous operands read half lines a stage:
 //     ahead from K = 1024 without a split (2000^3 33.8 -> 27.7), behind below
 //     (2048 x 3000 x 904 22.8 against 24.4) and split (333 x 777 x 5000 20.8
-//     against 22.9).
+//     against 22.9), and with one to two rounds of tiles, of which the
+//     register-staged kernel keeps three a CU (288 tiles, 3000 x 1500 x 2008 40.3
+//     against 44.1; 510, batch 3 of 1229 x 2064 x 3304 80.6 against 104.8; 576, 3000
+//     x 3000 x 2008 77.1 against 61.5 on wider tiles, which need 256 columns: 544,
+//     batch 16 of 4320 x 104 x 3304 180.8 against 197.8).
 bool edge_ring(const tvk_gemm_desc& d, const Plan& pl, int& tile) {
     if ((pl.kern != Kern::MFMA256W8 && pl.kern != Kern::MFMA128) || !pl.vec) return false;
-    if (pl.kern == Kern::MFMA128 && pl.ak && pl.bk && (pl.split > 1 || d.K < 1024)) return false;
+    if (pl.kern == Kern::MFMA128 && pl.ak && pl.bk) {
+        const int64_t t128 = ((d.M + 127) / 128) * ((d.N + 127) / 128) * d.batch;
+        if (pl.split > 1 || d.K < 1024 || (t128 > 256 && (t128 <= 512 || d.N < 256))) return false;
+    }
     const GemmArgs p = repacked_args(d, pl);
     if (dma_applies(p, pl.ak, pl.bk) || !dma_applies(p, pl.ak, pl.bk, true)) return false;
     const int64_t t256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * d.batch;
