@@ -25,16 +25,22 @@ def plan(m, n, k, batch=1):
 
 # (m, n, k, batch) the ring takes, and a neighbour across the line that it leaves to the tiles
 @pytest.mark.parametrize("ring,tiles", [
-    ((17, 512, 136, 1), (17, 512, 128, 1)),              # 8 k a row
-    ((32, 512, 256, 1), (32, 512, 248, 1)),
+    ((17, 512, 72, 1), (17, 512, 64, 1)),                # 4 k a row, 8 from 33 rows
+    ((32, 512, 128, 1), (32, 512, 120, 1)),
+    ((33, 512, 264, 1), (33, 512, 256, 1)),
     ((64, 512, 512, 1), (64, 512, 504, 1)),
     ((32, 16384, 1024, 1), (32, 16448, 1024, 1)),        # one round of workgroups
-    ((33, 14336, 1024, 1), (33, 14400, 1024, 1)),
+    ((33, 16384, 1024, 1), (33, 16448, 1024, 1)),
+    ((48, 32768, 1000, 1), (48, 32832, 1000, 1)),        # two, K off the 32 grid
+    ((24, 20000, 776, 1), (24, 20000, 744, 1)),
+    ((24, 20000, 2040, 1), (24, 20000, 2056, 1)),
     ((32, 32000, 4096, 1), (33, 32000, 4096, 1)),        # one long wide weight
     ((24, 1024, 512, 16), (24, 1024, 512, 17)),
-    ((64, 448, 1000, 32), (64, 512, 1000, 32)),
-    ((20, 64, 2048, 64), (20, 64, 2048, 65)),            # batches that the tiles split too
-    ((32, 512, 8192, 8), (32, 512, 8192, 16)),
+    ((64, 512, 1000, 32), (64, 576, 1000, 32)),
+    ((20, 64, 2048, 256), (20, 64, 2048, 257)),          # batches that the tiles split too
+    ((40, 64, 2048, 128), (40, 64, 2048, 129)),
+    ((40, 64, 4096, 64), (40, 64, 4096, 65)),
+    ((32, 512, 8184, 16), (32, 512, 8192, 16)),
     ((32, 4096, 8192, 1), (33, 4096, 8192, 1)),
     ((33, 250, 8000, 1), (33, 250, 8192, 1)),
 ])

@@ -36,8 +36,9 @@ def test_edges(gpu, m, n, k):
     assert want.abs().max() <= 256
     xd, wd = x.to(DEV), w.to(DEV)
     c = torch.full((m, n), 7, dtype=dtype, device=DEV)
-    # (below 8 k a row the tiles take more than 16 rows)
-    assert gpu.gemm_plan(xd, wd.t(), c).startswith("gemm16_skinny_bk" if m <= 16 or k >= 8 * m else "gemm16_mfma_64x64")
+    # (below 4 k a row, 8 from 33 rows, the tiles take more than 16 rows)
+    ring = m <= 16 or k >= (4 if m <= 32 else 8) * m
+    assert gpu.gemm_plan(xd, wd.t(), c).startswith("gemm16_skinny_bk" if ring else "gemm16_mfma_64x64")
     for _ in range(3):   # counters are left at zero
         _abi.gemm(xd, wd.t(), c)
     torch.cuda.synchronize()

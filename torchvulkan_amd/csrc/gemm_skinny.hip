@@ -349,12 +349,15 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
     const int kb = split ? z * p.k_chunk : 0;
     const int kend = split ? min(p.K, kb + p.k_chunk) : p.K;
     const int nk = (kend - kb + SKR_KST - 1) / SKR_KST;
+    __builtin_assume(nk > 0);   // (without it the loop is laid out behind the epilogue, and fetched cold)
     const int per = SERIAL ? p.k_chunk / SKR_KST : nk;   // stages of a chunk
-    // the stage that the s-th load brings: a chunk's stages from its workgroup's first one round
+    // the stage that the s-th load brings: a chunk's stages from its workgroup's first one round (found once where
+    // there is one chunk: per load its remainder added 0.4 us to 7 x 512 x 512)
+    auto first_of = [&](int n) { return p.sb[2] % 2048 == 0 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)n) : 0; };
+    const int rot = SERIAL ? 0 : first_of(nk);
     auto stage_at = [&](int s) {
         const int c0 = SERIAL ? s / per * per : 0, n = SERIAL ? min(per, nk - c0) : nk;
-        const int rot = p.sb[2] % 2048 == 0 ? (int)((blockIdx.x + blockIdx.x / 8) % (unsigned)n) : 0;
-        const int i = s - c0 + rot;
+        const int i = s - c0 + (SERIAL ? first_of(n) : rot);
         return c0 + (i >= n ? i - n : i);
     };
 
@@ -470,25 +473,31 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
 // K = 2048 the split 128x128 tiles). It runs one workgroup a CU, whose stages
 // are 256 k, so it wants about one round of workgroups and a whole stage:
 //   - M <= 16, K >= 256 (8 rows, 32 x 2048 x 64: 1.15x the other kernel's
-//     time, K = 128 1.07x, 256 0.92x), and up to 384 workgroups or K >= 1536
-//     (4 x 128256 x 256 1.22x, x 1024 1.03x, x 1536 0.87x).
-//   - above, K >= 8 M: a stage does the products of whole 16-row blocks, 4 of
-//     them from 33 rows (64 x 4096 x 256 1.12x, x 512 0.99x; 32 x 4096 x 128
-//     0.94x, 256 0.81x).
-//   - at most one round of workgroups, 224 with 4 row blocks (64 x 20000 x
-//     1024, 313 of them, 1.43x; batch 64 of 64 x 512 x 1000 1.29x; 256 of them
-//     1.07x) except over one long wide weight, where the tiles starve too (32
-//     x 32000 x 5000 0.66x).
-//   - batches split K less well: from K = 2048, where the tiles split too, up
-//     to 64 workgroups (batch 16 of 32 x 512 x 8192, 128 of them, 1.17x; 4 of
-//     32 x 1000 x 4096 0.81x).
+//     time, K = 128 1.07x, 256 0.92x), and up to 384 workgroups (1024 for one
+//     row: batch 64 of 1 x 512 x 512 0.79x, of 4 1.06x) or K >= 1536 (4 x 128256
+//     x 256 1.22x, x 1024 1.03x, x 1536 0.87x).
+//   - above, K >= 4 M, from 33 rows 8 M: a stage does the products of whole
+//     16-row blocks, 4 of them from there (64 x 4096 x 256 1.12x, x 512 0.99x; 32
+//     x 4096 x 64 1.02x, x 128 0.94x).
+//   - at most one round of workgroups (64 x 20000 x 1024, 313 of them, 1.43x;
+//     batch 64 of 64 x 512 x 1000 1.29x; 33 x 16384 x 1024, 256 of them, 0.70x),
+//     two over one weight with K off the 32 grid, which the tiles stage through
+//     registers (33 x 32000 x 1000 0.90x; from K = 2048 they split, x 5000 1.2x),
+//     and any number over one long wide weight up to 32 rows, where the tiles
+//     starve too (32 x 32000 x 5000 0.66x).
+//   - batches split K less well than the tiles, which do from K = 2048: above 32
+//     rows half a round there (batch 16 of 64 x 512 x 2048 1.03x, 256 of 64 x 64 x
+//     2048 1.15x; of 17 x 1000 0.76x) and a quarter from K = 4096, up to 32 rows a
+//     quarter from 8192 (batch 16 of 32 x 512 x 8192, 128 workgroups, 1.17x; 4 of
+//     17 x 4096 x 4096, 256, 0.85x).
 bool kring_pays(const GemmArgs& p) {
     const int64_t wgs = (int64_t)((p.N + SKR_NB - 1) / SKR_NB) * p.batch;
-    if (p.M <= 16) return p.K >= 256 && (wgs <= 384 || p.K >= 1536);
-    if (p.M > (p.K < 8192 ? 64 : 32) || p.K < 8 * p.M) return false;
-    if (p.batch > 1 && p.K >= 2048 && wgs > 64) return false;
-    if (p.M <= 32) return wgs <= 256 || (p.batch == 1 && p.K >= 4096);
-    return wgs <= 224;
+    if (p.M <= 16) return p.K >= 256 && (wgs <= (p.M == 1 ? 1024 : 384) || p.K >= 1536);
+    if (p.M > (p.K < 8192 ? 64 : 32) || p.K < (p.M <= 32 ? 4 : 8) * p.M) return false;
+    if (p.batch > 1 && p.M <= 32) return wgs <= (p.K >= 8192 ? 64 : 256);
+    if (p.batch > 1) return wgs <= (p.K >= 4096 ? 64 : p.K >= 2048 ? 128 : 256);
+    if (p.M <= 32 && p.K >= 4096) return true;
+    return wgs <= (p.K % 32 != 0 && p.K >= 768 && p.K < 2048 ? 512 : 256);
 }
 
 bool kring_applies(const GemmArgs& p, bool b_kmajor, bool vec) {
