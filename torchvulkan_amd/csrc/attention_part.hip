@@ -3,7 +3,7 @@
 // 128 columns with zeros past the head dim. They ran on the general VALU
 // kernels before (attention_any.hip), whose scores and products are scalar
 // fused multiply-adds over float32 LDS tiles: forward and backward of bfloat16
-// 8 x 16 heads x 577 x 80 took 4690 us there and take 172 us here. The next
+// 8 x 16 heads x 577 x 80 took 4690 us there and take 162 us here. The next
 // tile width above the head dim, since a column of zeros costs its products
 // and its LDS but no memory traffic.
 #include "attention_kernels.h"
