@@ -327,8 +327,6 @@ constexpr int SKR_B = SR_NW * 16 * SKR_K * 2;   // B bytes per stage: 32 KB, 4 K
 // LDS bytes of a stage (MF 16-row blocks of A) and ring depth in 160 KB
 constexpr int kring_stage(int mf) { return SKR_B + mf * SKR_KG * 4096; }
 constexpr int kring_depth(int mf) { return std::min(4, 160 * 1024 / kring_stage(mf)); }
-// and of the k halves' exchange, beside a ring of at most 3 stages where it recurs (SERIAL)
-constexpr int kring_red(int mf) { return SR_NW / SKR_KG * mf * 1024; }
 
 // SERIAL: one workgroup takes a strip's K chunks one after another, for calls
 // without memory for partials. It adds the chunks' sums in chunk order, the
@@ -336,11 +334,10 @@ constexpr int kring_red(int mf) { return SR_NW / SKR_KG * mf * 1024; }
 template <int DT, int MF, bool SERIAL>
 __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs p) {
     constexpr int CG = SR_NW / SKR_KG;   // 16-column groups
-    constexpr int NS = SERIAL ? std::min(3, kring_depth(MF)) : kring_depth(MF), STB = kring_stage(MF);
+    constexpr int NS = kring_depth(MF), STB = kring_stage(MF);
     constexpr int AL = 4 * MF * SKR_KG / SR_NW;   // A loads per wave
     static_assert(AL * SR_NW == 4 * MF * SKR_KG, "whole loads");
-    static_assert(NS * STB + (SERIAL ? kring_red(MF) : 0) <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(1024))) char lds_raw[NS * STB + (SERIAL ? kring_red(MF) : 0)];
+    __shared__ __attribute__((aligned(1024))) char lds_raw[NS * STB];
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(TVK_LDS char*)lds_raw);
     const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int cg = wave % CG, kg = wave / CG;
@@ -397,9 +394,9 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
     f32x4 acc[MF], total[MF];   // (total: SERIAL only)
 #pragma unroll
     for (int m = 0; m < MF; ++m) acc[m] = total[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // the second k half's sums onto the first's
-    f32x4* red = reinterpret_cast<f32x4*>(lds_raw + (SERIAL ? NS * STB : 0));
-    auto add_halves = [&]() {
+    // the second k half's sums onto the first's, through a ring slot that every wave has left
+    auto add_halves = [&](int slot) {
+        f32x4* red = reinterpret_cast<f32x4*>(lds_raw + slot * STB);
         if (kg > 0) {
 #pragma unroll
             for (int m = 0; m < MF; ++m) red[(cg * MF + m) * 64 + lane] = acc[m];
@@ -431,7 +428,8 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
             }
         }
         if (SERIAL && ((kt + 1) % per == 0 || kt == nk - 1)) {
-            add_halves();   // (read again after the next stage's barrier at the earliest)
+            __syncthreads();
+            add_halves(kt % NS);   // stage kt's slot, loaded again after the next stage's barrier
 #pragma unroll
             for (int m = 0; m < MF; ++m) {
                 total[m] = kt < per ? acc[m] : total[m] + acc[m];
@@ -445,7 +443,7 @@ __global__ __launch_bounds__(64 * SR_NW) void gemm_skinny_kring_kernel(GemmArgs 
 #pragma unroll
         for (int m = 0; m < MF; ++m) acc[m] = total[m];
     } else {
-        add_halves();
+        add_halves(0);
     }
 
     // lane l holds column l % 16 of the wave's 16, rows 16 m + (l / 16) * 4 + r
